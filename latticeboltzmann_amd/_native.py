@@ -156,6 +156,10 @@ SIGNATURES = {
                                   _vp, _vp, _vp]),
     "lbm_ghost_step_f32": (_i32, [_vp, _vp, _i64, _i64, _i32, _f64, _vp, _i32, _vp, _i32, _vp,
                                   _vp, _vp, _vp]),
+    "lbm_ghost_run_f64": (_i32, [_vp, _vp, _i64, _i64, _i32, _f64, _vp, _i32, _vp, _i64, _vp, _vp,
+                                 _vp, ctypes.POINTER(_i32), _vp]),
+    "lbm_ghost_run_f32": (_i32, [_vp, _vp, _i64, _i64, _i32, _f64, _vp, _i32, _vp, _i64, _vp, _vp,
+                                 _vp, ctypes.POINTER(_i32), _vp]),
 }
 
 _lib = None

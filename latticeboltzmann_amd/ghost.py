@@ -5,7 +5,7 @@ The reference's ``simulators/simple_flows`` and ``experimantal_flows``
 scripts keep one ghost layer inside the ``(9, nx, ny)`` array, stream it with
 ``np.roll``, overwrite populations next to the ghost layer and collide every
 node with their own equilibrium arithmetic (``PoiseuilleFlow.py:25-53``).
-``GhostLattice`` runs one such step per launch (``lbm_ghost_step_*``): the
+``GhostLattice`` runs up to four such steps per launch (``lbm_ghost_run_*``): the
 boundary handling of a script is a table of override rules (``Rule``) and an
 optional pressure-periodic pair of columns, and the kernel reproduces the
 script's arithmetic bit for bit in FP64 and FP32.
@@ -28,6 +28,7 @@ Drivers with the scripts' loops: ``couette`` (``PoiseuilleFlow.py:93-113``),
 """
 
 import ctypes
+import operator
 from dataclasses import dataclass
 
 import numpy as np
@@ -244,8 +245,17 @@ class GhostLattice:
     def step(self, n=1, moments=None):
         """n full steps (walls, then collide); ``moments`` receives the
         pre-collision moments of the last one."""
-        for s in range(n):
-            self._launch(0, moments if s == n - 1 else None)
+        n = operator.index(n)
+        if n > 0:
+            rho, ux, uy = moments if moments is not None else (None, None, None)
+            in_b = ctypes.c_int()
+            nat.call("lbm_ghost_run_" + _SUFFIX[self.dtype], nat.ptr(self.f), nat.ptr(self._g),
+                     self.nx, self.ny, self.layout, self.omega, ctypes.addressof(self._rules),
+                     len(self.rules),
+                     ctypes.addressof(self._pbc) if self._pbc is not None else None, n,
+                     nat.ptr(rho), nat.ptr(ux), nat.ptr(uy), ctypes.byref(in_b), nat.stream_ptr())
+            if in_b.value:
+                self.f, self._g = self._g, self.f
         self.time += n
         return self
 

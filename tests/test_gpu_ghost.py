@@ -146,3 +146,60 @@ def test_sliding_lid_reference_config(gpu):
     u = ux.cpu().numpy()
     assert np.isfinite(lat.populations()).all()
     assert u[151, -2] > 0.05 and u[151, 20:150].min() < 0  # lid-driven primary vortex
+
+
+@pytest.mark.parametrize("tdt,ndt", DT)
+@pytest.mark.parametrize("nx,ny,steps", [(24, 24, 9), (45, 67, 7), (45, 67, 6), (361, 1067, 5),
+                                         (352, 1058, 7)])
+@pytest.mark.parametrize("flow", ["lid", "couette", "poiseuille", "canal", "sides", "far"])
+def test_several_steps_per_launch_match_oracle(gpu, flow, tdt, ndt, nx, ny, steps):
+    # small-grid tiles and the two large-grid tiles, every remainder of the
+    # four steps a launch takes, wall tiles that are whole, cut, or one node
+    # wide; "far" has a rule that reads across many columns (single steps)
+    from latticeboltzmann_amd import ghost
+    print("multi", flow, tdt, nx, ny, steps, flush=True)
+    mx, my = nx // 2, ny // 2
+    ob = (mx, my - 2, mx + 3, my + 1)
+    rules, pbc, before, after = [], None, None, None
+    if flow == "lid":
+        rules = ghost.cavity_walls(nx, ny, 0.1)
+        after = lambda G: g.bounce_back_cavity(G, 0.1)
+    elif flow == "couette":
+        rules = ghost.channel_walls(nx, ny, 0.1)
+        after = lambda G: g.bounce_back_channel(G, 0.1)
+    elif flow == "poiseuille":
+        rules, pbc = ghost.channel_walls(nx, ny, 0.02), ("before", 1.01, 0.99)
+        before = lambda G: g.pressure_periodic(G, 1.01, 0.99)
+        after = lambda G: g.bounce_back_channel(G, 0.02)
+    elif flow == "canal":
+        rules = ghost.side_walls(nx, ny, 0.05) + ghost.obstacle_faces(*ob)
+        pbc = ("after", 1.01, 0.99)
+
+        def after(G):
+            g.pressure_periodic_after(G, 1.01, 0.99)
+            g.bounce_back_walls(G, 0.05)
+            g.apply_obstacle(G, *ob)
+    elif flow == "sides":
+        rules = ghost.side_walls(nx, ny, left=True, right=True, bottom=False, top=False)
+        after = lambda G: g.bounce_back_walls(G, 0.0, left=True, right=True, bottom=False, top=False)
+    else:
+        rules = [ghost.Rule(3, 5, 2, 9, 1, 3, nx - 6, 4)]
+
+        def after(G):
+            G[1, 3:5, 2:9] = G[3, nx - 3:nx - 1, 6:13]
+    r = np.random.default_rng(nx + steps)
+    rho = (1 + 0.02 * r.standard_normal((nx, ny))).astype(ndt)
+    ux, uy = ((0.03 * r.standard_normal((nx, ny))).astype(ndt) for _ in range(2))
+    lat = ghost.GhostLattice(nx, ny, 1.3, rules, pbc, dtype=tdt,
+                             layout="soa" if steps == 6 else "rows")
+    lat.init_equilibrium(rho, ux, uy)
+    mom = lat.moment_buffers()
+    lat.step(steps, moments=mom)
+    G = g.equilibrium(rho, ux, uy)
+    for _ in range(steps):
+        if before:
+            before(G)
+        g.stream(G)
+        after(G)
+        omom = g.collide(G, 1.3)
+    same(lat, mom, G, omom)
