@@ -362,11 +362,18 @@ int lbm_nn_gemm(const void *A, int64_t sam, int64_t sak, const void *B, int64_t 
  *             flip_weights (wf[tap][co][c] = w[co][tap*cin + c]).               */
 int lbm_nn_conv3x3(const void *x, int B, int H, int W, int cin, const void *w, int cout,
                    const float *bias, float *y, void *yb, int relu, void *stream);
+/* pixel splits that fill the GPU (the workspace is that of a GEMM so split) */
+int lbm_nn_conv3x3_wgrad_splits(int B, int H, int W, int cin, int cout);
 int lbm_nn_conv3x3_wgrad(const void *x, const void *dy, int B, int H, int W, int cin, int cout,
                          float *dw, int ksplit, float *work, void *stream);
 int lbm_nn_conv3x3_flip_weights(const void *w, int cin, int cout, void *wf, void *stream);
 int lbm_nn_conv3x3_dgrad(const void *dy, const void *wf, int B, int H, int W, int cin, int cout,
                          float *dx, int accumulate, void *stream);
+/* The same from weights in wt[cin][tap][cout] (lbm_nn_conv3x3_transpose_weights):
+ * k contiguous, which the direct kernel (cout a multiple of 32) loads as it is. */
+int lbm_nn_conv3x3_transpose_weights(const void *w, int cin, int cout, void *wt, void *stream);
+int lbm_nn_conv3x3_dgrad_t(const void *dy, const void *wt, int B, int H, int W, int cin, int cout,
+                           float *dx, int accumulate, void *stream);
 /* cols[((b*H + y)*W + x)*9*C + (dy*3 + dx)*C + c] = x[b][y+dy-1][x+dx-1][c] (0 outside). */
 int lbm_nn_im2col3x3(const void *x, int B, int H, int W, int C, void *cols, void *stream);
 /* Adjoint of im2col3x3 (a gather, FP32): dx (+)= col2im(dcols).              */

@@ -131,8 +131,11 @@ SIGNATURES = {
                            _i32, _i32, _i32, _i32, _vp, _vp]),
     "lbm_nn_conv3x3": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _i32, _vp, _vp, _vp, _i32, _vp]),
     "lbm_nn_conv3x3_wgrad": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _i32, _vp, _vp]),
+    "lbm_nn_conv3x3_wgrad_splits": (_i32, [_i32, _i32, _i32, _i32, _i32]),
     "lbm_nn_conv3x3_flip_weights": (_i32, [_vp, _i32, _i32, _vp, _vp]),
     "lbm_nn_conv3x3_dgrad": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _i32, _vp]),
+    "lbm_nn_conv3x3_transpose_weights": (_i32, [_vp, _i32, _i32, _vp, _vp]),
+    "lbm_nn_conv3x3_dgrad_t": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _i32, _vp]),
     "lbm_nn_im2col3x3": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp]),
     "lbm_nn_col2im3x3": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _i32, _vp]),
     "lbm_nn_relu_backward": (_i32, [_vp, _vp, _vp, _i64, _vp]),

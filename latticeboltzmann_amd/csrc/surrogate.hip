@@ -238,6 +238,318 @@ __global__ __launch_bounds__(256) void k_gemm_reduce(GemmArgs g, int splits) {
     if (g.Cb) g.Cb[o] = f2bf(v);
 }
 
+// ---------------------------------------------------------------------------
+// 3x3 same convolution with C % 32 == 0 input channels: out[p][n] = sum over
+// taps and c of X[p + sign * tap][c] W[n][tap * C + c], NHWC BF16, FP32
+// accumulation in the k order of k_gemm (tap by tap, 32 channels a step), so
+// the results are its bits.  sign +1: forward; -1: data gradient.
+//
+// Both MFMA operands want 8 consecutive channels of one row per lane, which is
+// how X and W lie in memory, so every lane loads its fragments straight into
+// registers (16 bytes each): no LDS, no barrier, D steps of loads in flight per
+// wave.  (k_gemm moves each step's tiles through LDS between two barriers with
+// nothing in flight: about 1 us per step, whatever the step computes.)  Pixels
+// outside the image are loaded from an offset past the buffer's end, which the
+// buffer load answers with zeros.  The weights are the MFMA's row operand, so a
+// lane ends with 4 consecutive output channels of one pixel: 16-byte stores.
+// A wave computes MT x 16 pixels x NT x 16 channels; the 4 waves of a block
+// take consecutive pixels and share the weights through L1.
+struct ConvArgs {
+    const uint16_t *X, *Wt;
+    float *y;      // nullable
+    uint16_t *yb;  // nullable
+    const float *bias;
+    int P, H, W, C, N, sign, accumulate, relu;
+};
+
+template <int MT, int NT, int D>
+__global__ __launch_bounds__(256) void k_conv3(ConvArgs a) {
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(int(blockIdx.x * 4 + (threadIdx.x >> 6)));
+    const int p0 = wave * 16 * MT, n0 = blockIdx.y * 16 * NT;
+    if (p0 >= a.P) return;
+    const int col = lane & 15, kq = (lane >> 4) * 8;
+    const unsigned xbytes = unsigned(a.P) * unsigned(a.C) * 2u;
+    const unsigned wbytes = unsigned(a.N) * 9u * unsigned(a.C) * 2u;
+    __amdgpu_buffer_rsrc_t xr =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(a.X), 0, int(xbytes), 0x00020000);
+    __amdgpu_buffer_rsrc_t wr =
+        __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t *>(a.Wt), 0, int(wbytes), 0x00020000);
+    constexpr unsigned kOutside = 0x80000000u;  // past any operand (host: below 2^31 bytes)
+
+    unsigned xo[MT];   // byte offset of the lane's pixel
+    unsigned in[MT];   // bit `tap`: the tap's pixel lies in the image
+    unsigned wo[NT];   // byte offset of the lane's weight row
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int p = p0 + m * 16 + col;
+        const int x = p % a.W, y = (p / a.W) % a.H;
+        unsigned bits = 0;
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap) {
+            const int yy = y + a.sign * (tap / 3 - 1), xx = x + a.sign * (tap % 3 - 1);
+            bits |= unsigned(p < a.P && unsigned(yy) < unsigned(a.H) && unsigned(xx) < unsigned(a.W)) << tap;
+        }
+        in[m] = bits;
+        xo[m] = (unsigned(p) * unsigned(a.C) + unsigned(kq)) * 2u;
+    }
+#pragma unroll
+    for (int n = 0; n < NT; ++n) {
+        const int r = n0 + n * 16 + col;
+        wo[n] = r < a.N ? (unsigned(r) * 9u * unsigned(a.C) + unsigned(kq)) * 2u : kOutside;
+    }
+
+    floatx4 acc[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+
+    const int per_tap = a.C / 32, S = 9 * per_tap;  // S is a multiple of D
+    u32x4 fx[D][MT], fw[D][NT];
+    int tap = 0, cc = 0, step = 0;  // of the next load
+    auto load = [&](u32x4 *bx, u32x4 *bw) {
+        const int shift = a.sign * ((tap / 3 - 1) * a.W + (tap % 3 - 1)) * a.C * 2 + cc * 64;
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const unsigned o = (in[m] >> tap) & 1u ? xo[m] + unsigned(shift) : kOutside;
+            bx[m] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, int(o), 0, 0));
+        }
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+            bw[n] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(
+                                                  wr, int(wo[n]), step * 64, 0));
+        ++step;
+        if (++cc == per_tap) cc = 0, ++tap;
+    };
+#pragma unroll
+    for (int d = 0; d < D; ++d) load(fx[d], fw[d]);
+    for (int s = 0; s < S; s += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                        __builtin_bit_cast(bf16x8, fw[d][n]), __builtin_bit_cast(bf16x8, fx[d][m]),
+                        acc[m][n], 0, 0, 0);
+            if (s + D < S) load(fx[d], fw[d]);
+        }
+    }
+
+    const bool vec = (a.N & 3) == 0;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int p = p0 + m * 16 + col;
+        if (p >= a.P) continue;
+#pragma unroll
+        for (int n = 0; n < NT; ++n) {
+            const int c = n0 + n * 16 + (lane >> 4) * 4;
+            const int64_t o = int64_t(p) * a.N + c;
+            floatx4 v = acc[m][n];
+            if (vec) {
+                if (c >= a.N) continue;
+                if (a.accumulate) v += *reinterpret_cast<const floatx4 *>(a.y + o);
+                if (a.bias) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] += a.bias[c + r];
+                }
+                if (a.relu) {
+#pragma unroll
+                    for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.0f);
+                }
+                if (a.y) *reinterpret_cast<floatx4 *>(a.y + o) = v;
+                if (a.yb) {
+                    ushort4 h = make_ushort4(f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3]));
+                    *reinterpret_cast<ushort4 *>(a.yb + o) = h;
+                }
+                continue;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                if (c + r >= a.N) continue;
+                float u = v[r];
+                if (a.accumulate) u += a.y[o + r];
+                if (a.bias) u += a.bias[c + r];
+                if (a.relu) u = fmaxf(u, 0.0f);
+                if (a.y) a.y[o + r] = u;
+                if (a.yb) a.yb[o + r] = f2bf(u);
+            }
+        }
+    }
+}
+
+// Weight gradient of the 3x3 convolution: dW[co][tap * C + c] = sum over pixels
+// of dY[p][co] X[p + tap][c].  Here the MFMA's k is the pixel, and both operands
+// lie channel by channel, so a block stages 128 pixels at a time in LDS with
+// pixels and channels exchanged: a thread loads 8 pixels x 8 channels (16 bytes
+// each), exchanges them in registers and writes 8 x 16 bytes, instead of one
+// 2-byte LDS store per element.  A block owns 16 MT output channels, 32 input
+// channels and the three taps of one row dy; X is staged once per dx with the
+// pixels outside the image as zeros, so every fragment is an aligned 16-byte
+// LDS read.  Each wave takes a quarter of the staged pixels and the whole tile
+// (MT x 6 MFMAs from MT + 6 reads a step); the four waves' sums are added in
+// order at the end.  The next 128 pixels' loads are in flight meanwhile.
+struct WgradArgs {
+    const uint16_t *X, *dY;
+    float *out;  // dW, or the split's partial sums
+    int P, H, W, C, N, chunk;
+};
+
+// 8 consecutive channels of one row at byte offset o; channels >= n (n <= 8) and
+// rows at kOutside read as zero.  mode: 2 16-byte rows, 1 even row length, 0 any.
+__device__ __forceinline__ uint4 load_channels(__amdgpu_buffer_rsrc_t r, unsigned o, int n, int mode) {
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    if (mode == 2) {
+        const u32x4 v = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(r, int(o), 0, 0));
+        return make_uint4(v.x, v.y, v.z, v.w);
+    }
+    unsigned v[4] = {0, 0, 0, 0};
+    if (o & 0x80000000u) return make_uint4(0, 0, 0, 0);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        if (mode == 1) {
+            if (2 * i < n) v[i] = unsigned(__builtin_amdgcn_raw_buffer_load_b32(r, int(o) + 4 * i, 0, 0));
+        } else {
+            if (2 * i < n) v[i] = uint16_t(__builtin_amdgcn_raw_buffer_load_b16(r, int(o) + 4 * i, 0, 0));
+            if (2 * i + 1 < n)
+                v[i] |= unsigned(uint16_t(__builtin_amdgcn_raw_buffer_load_b16(r, int(o) + 4 * i + 2, 0, 0))) << 16;
+        }
+    }
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
+
+constexpr int kWgradPx = 128;
+constexpr int64_t WGRAD_BLOCKS = 3;
+
+template <int MT>
+__global__ __launch_bounds__(256) void k_wgrad(WgradArgs a) {
+    constexpr int CO = 16 * MT, PITCH = kWgradPx + 8, G = kWgradPx / 8;
+    constexpr int kA = G * CO / 8, kB = 3 * G * 4, R = (kA + kB + 255) / 256;
+    constexpr unsigned kOutside = 0x80000000u;
+    constexpr int kStage = (CO + 96) * PITCH * 2, kSums = 4 * 6 * 256 * 4;
+    __shared__ __align__(16) unsigned char smem[kStage > kSums ? kStage : kSums];
+    uint16_t *const sA = reinterpret_cast<uint16_t *>(smem);  // [CO][PITCH]
+    uint16_t *const sB = sA + CO * PITCH;                     // [3][32][PITCH]
+    const int t = threadIdx.x, lane = t & 63, w = t >> 6, col = lane & 15;
+    // block: (co tile, c tile, dy) of blockIdx.x
+    const int nc = (a.C + 31) / 32;
+    int b = blockIdx.x;
+    const int dy = b % 3 - 1;
+    b /= 3;
+    const int c0 = (b % nc) * 32, co0 = (b / nc) * CO;
+    const int beg = blockIdx.y * a.chunk, end = min(a.P, beg + a.chunk);
+
+    __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t *>(a.X), 0, int(unsigned(a.P) * unsigned(a.C) * 2u), 0x00020000);
+    __amdgpu_buffer_rsrc_t yr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t *>(a.dY), 0, int(unsigned(a.P) * unsigned(a.N) * 2u), 0x00020000);
+    const int mx = a.C % 8 == 0 ? 2 : (a.C % 2 == 0 ? 1 : 0), my = a.N % 8 == 0 ? 2 : (a.N % 2 == 0 ? 1 : 0);
+
+    uint4 r[R][8];
+    auto fetch = [&](int pb) {
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const int it = t + q * 256;
+            if (it < kA) {
+                const int g = it / (CO / 8), ch = co0 + (it % (CO / 8)) * 8;
+                const int p = pb + g * 8;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const bool in = p + j < end && ch < a.N;
+                    const unsigned o = in ? (unsigned(p + j) * unsigned(a.N) + unsigned(ch)) * 2u : kOutside;
+                    r[q][j] = load_channels(yr, o, a.N - ch, my);
+                }
+            } else if (it < kA + kB) {
+                const int i = it - kA, dx = i / (G * 4) - 1, g = (i / 4) % G, ch = c0 + (i % 4) * 8;
+                const int p = pb + g * 8;
+                int x = p % a.W, y = (p / a.W) % a.H;
+#pragma unroll
+                for (int j = 0; j < 8; ++j) {
+                    const bool in = p + j < end && ch < a.C && unsigned(x + dx) < unsigned(a.W) &&
+                                    unsigned(y + dy) < unsigned(a.H);
+                    const unsigned o =
+                        in ? (unsigned(p + j + dy * a.W + dx) * unsigned(a.C) + unsigned(ch)) * 2u : kOutside;
+                    r[q][j] = load_channels(xr, o, a.C - ch, mx);
+                    if (++x == a.W) {
+                        x = 0;
+                        if (++y == a.H) y = 0;
+                    }
+                }
+            }
+        }
+    };
+    auto stage = [&]() {
+#pragma unroll
+        for (int q = 0; q < R; ++q) {
+            const int it = t + q * 256;
+            if (it >= kA + kB) continue;
+            uint16_t *d;  // row of the item's first channel
+            if (it < kA) d = sA + (it % (CO / 8)) * 8 * PITCH + (it / (CO / 8)) * 8;
+            else d = sB + ((it - kA) / (G * 4) * 32 + ((it - kA) % 4) * 8) * PITCH + ((it - kA) / 4 % G) * 8;
+            const unsigned *v = reinterpret_cast<const unsigned *>(r[q]);
+#pragma unroll
+            for (int c = 0; c < 8; ++c) {
+                // channel c of pixels 2i and 2i + 1
+                unsigned o[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+                    o[i] = __builtin_amdgcn_perm(v[(2 * i + 1) * 4 + c / 2], v[2 * i * 4 + c / 2],
+                                                 c % 2 ? 0x07060302u : 0x05040100u);
+                *reinterpret_cast<uint4 *>(d + c * PITCH) = make_uint4(o[0], o[1], o[2], o[3]);
+            }
+        }
+    };
+
+    floatx4 acc[MT][6];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < 6; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+    const int k = w * 32 + (lane >> 4) * 8;  // the lane's pixels of a stage
+    fetch(beg);
+    for (int pb = beg; pb < end; pb += kWgradPx) {
+        stage();
+        __syncthreads();
+        if (pb + kWgradPx < end) fetch(pb + kWgradPx);
+        bf16x8 x[6];
+#pragma unroll
+        for (int n = 0; n < 6; ++n)  // n = 2 dx + c tile
+            x[n] = *reinterpret_cast<const bf16x8 *>(sB + (n * 16 + col) * PITCH + k);
+#pragma unroll
+        for (int m = 0; m < MT; ++m) {
+            const bf16x8 y = *reinterpret_cast<const bf16x8 *>(sA + (m * 16 + col) * PITCH + k);
+#pragma unroll
+            for (int n = 0; n < 6; ++n)
+                acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(y, x[n], acc[m][n], 0, 0, 0);
+        }
+        __syncthreads();
+    }
+
+    float *const sums = reinterpret_cast<float *>(smem);  // [wave][n][16 x 16]
+    float *const out = a.out + int64_t(blockIdx.y) * a.N * 9 * a.C;
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+#pragma unroll
+        for (int n = 0; n < 6; ++n)
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+                sums[(w * 6 + n) * 256 + ((lane >> 4) * 4 + i) * 16 + col] = acc[m][n][i];
+        __syncthreads();
+#pragma unroll
+        for (int n = 0; n < 6; ++n) {
+            const float v = ((sums[n * 256 + t] + sums[(6 + n) * 256 + t]) + sums[(12 + n) * 256 + t]) +
+                            sums[(18 + n) * 256 + t];
+            const int co = co0 + m * 16 + (t >> 4), c = c0 + (n & 1) * 16 + (t & 15);
+            if (co < a.N && c < a.C)
+                out[(int64_t(co) * 9 + (dy + 1) * 3 + n / 2) * a.C + c] = v;
+        }
+        __syncthreads();
+    }
+}
+
 // im2col for 3x3 same convolution: x [B][H][W][C] BF16 -> cols [B*H*W][9*C].
 // Tap (dy, dx) = (blockIdx.y / 3, blockIdx.y % 3); each thread moves VEC
 // consecutive channels of one pixel (VEC = 8: one 16-byte load and store,
@@ -334,6 +646,17 @@ __global__ __launch_bounds__(256) void k_bias_grad_final(const double *__restric
     const double v = t < nblocks ? partial[int64_t(t) * N + n] : 0.0;
     const double tot = block_sum(v);
     if (t == 0) db[n] = float(tot);
+}
+
+// Weights W[cout][tap][cin] -> Wt[cin][tap][cout] (BF16): the weights of the data
+// gradient as a convolution of dY, k contiguous.
+__global__ __launch_bounds__(256) void k_transpose_weights(const uint16_t *__restrict__ w, int cin,
+                                                           int cout, uint16_t *__restrict__ wt) {
+    const int i = blockIdx.x * 256 + threadIdx.x;  // over cin, tap, cout
+    if (i >= 9 * cout * cin) return;
+    const int co = i % cout, r = i / cout;
+    const int tap = r % 9, c = r / 9;
+    wt[i] = w[(int64_t(co) * 9 + tap) * cin + c];
 }
 
 // Weights W[cout][tap][cin] -> Wf[tap][cout][cin] (BF16): the B operand of the
@@ -698,6 +1021,45 @@ static int run_gemm(const GemmArgs &g, int splits, hipStream_t s) {
     return launch_status();
 }
 
+// k_conv3 where it applies: C a multiple of the 32 channels of a step, 16-byte
+// aligned operands and (vector stores) outputs, operands below 2^31 bytes.
+static bool conv_direct(const ConvArgs &a) {
+    auto misaligned = [](const void *q) { return reinterpret_cast<uintptr_t>(q) % 16 != 0; };
+    if (a.C % 32 || misaligned(a.X) || misaligned(a.Wt) || misaligned(a.y) || misaligned(a.yb)) return false;
+    return int64_t(a.P) * a.C * 2 < (int64_t(1) << 31) && int64_t(a.N) * 9 * a.C * 2 < (int64_t(1) << 31);
+}
+
+// Output channels of a k_wgrad block: 64 where they divide evenly, else 32 (the
+// staged X is shared by half as many, but none are computed for nothing).
+static int wgrad_co(int cout) { return cout % 64 == 0 ? 64 : 32; }
+
+// k_wgrad where its loads apply: offsets below 2^31 bytes, rows that are a multiple
+// of 16 bytes on a 16-byte base, others on a 4-byte one.
+static bool wgrad_direct(const void *x, const void *dy, int64_t P, int cin, int cout) {
+    auto ok = [&](const void *q, int n) {
+        return reinterpret_cast<uintptr_t>(q) % (n % 8 == 0 ? 16 : 4) == 0 && P * n * 2 < (int64_t(1) << 31);
+    };
+    return ok(x, cin) && ok(dy, cout);
+}
+
+static int run_conv(const ConvArgs &a, hipStream_t s) {
+    // The largest tile that still gives every SIMD two waves: operands loaded per
+    // MFMA fall with the tile, but a wave's 9 C / 32 steps are a serial chain.
+    const int64_t simds = 4 * int64_t(device_cus());
+    auto waves = [&](int mt, int nt) {
+        return int64_t((a.P + 16 * mt - 1) / (16 * mt)) * ((a.N + 16 * nt - 1) / (16 * nt));
+    };
+    auto launch = [&](auto kernel, int mt, int nt) {
+        const dim3 grid(unsigned((a.P + 64 * mt - 1) / (64 * mt)), unsigned((a.N + 16 * nt - 1) / (16 * nt)));
+        hipLaunchKernelGGL(kernel, grid, dim3(256), 0, s, a);
+    };
+    if (a.N > 32 && waves(4, 4) >= 2 * simds) launch(k_conv3<4, 4, 3>, 4, 4);
+    else if (a.N > 16 && waves(4, 2) >= 2 * simds) launch(k_conv3<4, 2, 3>, 4, 2);
+    else if (a.N > 16 && waves(2, 2) >= 2 * simds) launch(k_conv3<2, 2, 3>, 2, 2);
+    else launch(k_conv3<1, 1, 9>, 1, 1);
+    return launch_status();
+}
+
 extern "C" {
 
 int64_t lbm_nn_gemm_workspace(int M, int N, int ksplit) {
@@ -728,12 +1090,25 @@ int lbm_nn_conv3x3(const void *x, int B, int H, int W, int cin, const void *w, i
     const int64_t P = int64_t(B) * H * W;
     if (P * 9 * cin >= (int64_t(1) << 31) || P * cout >= (int64_t(1) << 31)) return LBM_E_SIZE;
     if (cin % 8 == 0 && reinterpret_cast<uintptr_t>(x) % 16) return LBM_E_ARG;
+    const ConvArgs a{static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(w), y,
+                     static_cast<uint16_t *>(yb), bias, int(P), H, W, cin, cout, 1, 0, relu};
+    if (conv_direct(a)) return run_conv(a, as_stream(stream));
     const int K = 9 * cin;
     GemmArgs g{static_cast<const uint16_t *>(x), 0, 0, static_cast<const uint16_t *>(w), 1, K, y,
                static_cast<uint16_t *>(yb), cout, bias, int(P), cout, K, (K + TK - 1) / TK * TK, 0,
                relu, nullptr, LOAD_SCALAR, load_mode(w, K, 1), Gather{H, W, cin, 1},
                Gather{1, 1, 1, 0}};
     return run_gemm(g, 1, as_stream(stream));
+}
+
+int lbm_nn_conv3x3_wgrad_splits(int B, int H, int W, int cin, int cout) {
+    if (B <= 0 || H <= 0 || W <= 0 || cin <= 0 || cout <= 0) return LBM_E_SIZE;
+    const int64_t P = int64_t(B) * H * W, chunks = (P + kWgradPx - 1) / kWgradPx;
+    const int64_t co = wgrad_co(cout);
+    const int64_t tiles = 3 * ((cin + 31) / 32) * ((cout + co - 1) / co);
+    int64_t splits = (WGRAD_BLOCKS * int64_t(device_cus()) + tiles - 1) / tiles;
+    if (splits > (chunks + 3) / 4) splits = (chunks + 3) / 4;
+    return int(splits < 1 ? 1 : splits);
 }
 
 int lbm_nn_conv3x3_wgrad(const void *x, const void *dy, int B, int H, int W, int cin, int cout,
@@ -746,8 +1121,24 @@ int lbm_nn_conv3x3_wgrad(const void *x, const void *dy, int B, int H, int W, int
     if (ksplit > 1 && !work) return LBM_E_WORKSPACE;
     const int K = int(P), N = 9 * cin;
     int kchunk = (K + ksplit - 1) / ksplit;
-    kchunk = (kchunk + TK - 1) / TK * TK;
+    const int unit = P >= 2 * kWgradPx && wgrad_direct(x, dy, P, cin, cout) ? kWgradPx : TK;
+    kchunk = (kchunk + unit - 1) / unit * unit;
     const int splits = (K + kchunk - 1) / kchunk;
+    if (unit == kWgradPx) {
+        WgradArgs a{static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(dy),
+                    splits > 1 ? work : dw, K, H, W, cin, cout, kchunk};
+        const int co = wgrad_co(cout);
+        const dim3 grid(unsigned(3 * ((cin + 31) / 32) * ((cout + co - 1) / co)), unsigned(splits));
+        hipStream_t s = as_stream(stream);
+        if (co == 64) hipLaunchKernelGGL(k_wgrad<4>, grid, dim3(256), 0, s, a);
+        else hipLaunchKernelGGL(k_wgrad<2>, grid, dim3(256), 0, s, a);
+        if (splits > 1) {
+            GemmArgs g{};
+            g.C = dw, g.ldc = N, g.M = cout, g.N = N, g.work = work;
+            hipLaunchKernelGGL(k_gemm_reduce, dim3(blocks_for(int64_t(cout) * N)), dim3(256), 0, s, g, splits);
+        }
+        return launch_status();
+    }
     GemmArgs g{static_cast<const uint16_t *>(dy), 1, cout, static_cast<const uint16_t *>(x), 0, 0,
                dw, nullptr, N, nullptr, cout, N, K, kchunk, 0, 0, work, load_mode(dy, 1, cout),
                LOAD_SCALAR, Gather{1, 1, 1, 0}, Gather{H, W, cin, 1}};
@@ -774,6 +1165,33 @@ int lbm_nn_conv3x3_dgrad(const void *dy, const void *wf, int B, int H, int W, in
     GemmArgs g{static_cast<const uint16_t *>(dy), 0, 0, static_cast<const uint16_t *>(wf), cin, 1,
                dx, nullptr, cin, nullptr, int(P), cin, K, (K + TK - 1) / TK * TK, accumulate, 0,
                nullptr, LOAD_SCALAR, load_mode(wf, 1, cin), Gather{H, W, cout, -1},
+               Gather{1, 1, 1, 0}};
+    return run_gemm(g, 1, as_stream(stream));
+}
+
+int lbm_nn_conv3x3_transpose_weights(const void *w, int cin, int cout, void *wt, void *stream) {
+    if (!w || !wt) return LBM_E_NULL;
+    if (cin <= 0 || cout <= 0) return LBM_E_SIZE;
+    hipLaunchKernelGGL(k_transpose_weights, dim3(blocks_for(int64_t(9) * cout * cin)), dim3(256), 0,
+                       as_stream(stream), static_cast<const uint16_t *>(w), cin, cout,
+                       static_cast<uint16_t *>(wt));
+    return launch_status();
+}
+
+int lbm_nn_conv3x3_dgrad_t(const void *dy, const void *wt, int B, int H, int W, int cin, int cout,
+                           float *dx, int accumulate, void *stream) {
+    if (!dy || !wt || !dx) return LBM_E_NULL;
+    if (B <= 0 || H <= 0 || W <= 0 || cin <= 0 || cout <= 0) return LBM_E_SIZE;
+    const int64_t P = int64_t(B) * H * W;
+    if (P * 9 * cout >= (int64_t(1) << 31) || P * cin >= (int64_t(1) << 31)) return LBM_E_SIZE;
+    if (cout % 8 == 0 && reinterpret_cast<uintptr_t>(dy) % 16) return LBM_E_ARG;
+    const ConvArgs a{static_cast<const uint16_t *>(dy), static_cast<const uint16_t *>(wt), dx, nullptr,
+                     nullptr, int(P), H, W, cout, cin, -1, accumulate, 0};
+    if (conv_direct(a)) return run_conv(a, as_stream(stream));
+    const int K = 9 * cout;
+    GemmArgs g{static_cast<const uint16_t *>(dy), 0, 0, static_cast<const uint16_t *>(wt), 1, K,
+               dx, nullptr, cin, nullptr, int(P), cin, K, (K + TK - 1) / TK * TK, accumulate, 0,
+               nullptr, LOAD_SCALAR, load_mode(wt, K, 1), Gather{H, W, cout, -1},
                Gather{1, 1, 1, 0}};
     return run_gemm(g, 1, as_stream(stream));
 }

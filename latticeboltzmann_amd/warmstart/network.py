@@ -176,10 +176,6 @@ class Surrogate:
         out, _ = conv("head", h, hb)
         return (out, cache) if keep else out
 
-    def _ksplit(self, cout, K, P):
-        base = -(-K // 64) * -(-cout // 64)
-        return max(1, min(64, -(-1024 // base), P // 512))
-
     def _back(self, cache, name, dy, need_dx=True):
         xb, y, (B, H, W, cin) = cache[name]
         _, cout, relu = self.spec[name]
@@ -192,7 +188,7 @@ class Surrogate:
         else:
             nat.call("lbm_nn_to_bf16", _p(dy), _p(dyb), dy.numel(), s)
         gw, gbias = self.views(name, self.g)
-        ks = self._ksplit(cout, K, P)
+        ks = int(nat.load().lbm_nn_conv3x3_wgrad_splits(B, H, W, cin, cout))
         work = None
         if ks > 1:
             work = torch.empty(int(nat.load().lbm_nn_gemm_workspace(cout, K, ks)) // 4,
@@ -208,9 +204,9 @@ class Surrogate:
         # dx[p][c] = sum over taps and co of dy[p - tap][co] W[co][tap][c]
         wb = self.views(name, self.pb)[0]
         wf = torch.empty(9 * cin * cout, dtype=torch.bfloat16, device=self.device)
-        nat.call("lbm_nn_conv3x3_flip_weights", _p(wb), cin, cout, _p(wf), s)
+        nat.call("lbm_nn_conv3x3_transpose_weights", _p(wb), cin, cout, _p(wf), s)
         dx = torch.empty((B, H, W, cin), dtype=torch.float32, device=self.device)
-        nat.call("lbm_nn_conv3x3_dgrad", _p(dyb), _p(wf), B, H, W, cin, cout, _p(dx), 0, s)
+        nat.call("lbm_nn_conv3x3_dgrad_t", _p(dyb), _p(wf), B, H, W, cin, cout, _p(dx), 0, s)
         return dx
 
     def backward(self, cache, dout, need_input_grad=False):

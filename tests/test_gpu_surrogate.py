@@ -474,3 +474,50 @@ def test_parameter_average_kernel(gpu):
     want = 0.99 * e0.double() + 0.01 * p.double()
     assert float((ema.double() - want).abs().max()) < 1e-6
     assert nat.load().lbm_nn_ema(_p(ema), _p(p), 1000, 1.0, nat.stream_ptr()) == -3
+
+
+# (B, H, W, cin, cout): ragged pixel tiles, images narrower than a tile, output
+# channels that fill no tile, weight-gradient channel tiles of 3 and 18, and
+# sizes that reach each of the direct kernel's tiles
+@pytest.mark.parametrize("B,H,W,cin,cout", [(1, 16, 17, 32, 3), (3, 9, 11, 64, 96), (2, 16, 20, 18, 32),
+                                            (2, 13, 10, 96, 40), (5, 72, 90, 32, 32), (9, 64, 64, 64, 128)])
+def test_conv3x3_direct_kernels(gpu, B, H, W, cin, cout):
+    nat = _nat()
+    rng = np.random.default_rng(cin + cout)
+    P, K, sp, lib = B * H * W, 9 * cin, nat.stream_ptr(), nat.load()
+    x, _ = _bf(rng, (B, H, W, cin))
+    w, _ = _bf(rng, (cout, 3, 3, cin), 0.2)
+    dy, _ = _bf(rng, (B, H, W, cout))
+    bias = torch.as_tensor(rng.normal(size=cout).astype(np.float32)).cuda()
+    cols = torch.empty((P, K), dtype=torch.bfloat16, device="cuda")
+    nat.call("lbm_nn_im2col3x3", _p(x), B, H, W, cin, _p(cols), sp)
+    # forward: the k order of im2col + GEMM, so its bits
+    ye, yeb = (torch.empty((P, cout), dtype=t, device="cuda") for t in (torch.float32, torch.bfloat16))
+    nat.call("lbm_nn_gemm", _p(cols), K, 1, _p(w), 1, K, _p(ye), _p(yeb), cout, _p(bias),
+             P, cout, K, 0, 1, 1, None, sp)
+    y, yb = torch.empty_like(ye), torch.empty_like(yeb)
+    nat.call("lbm_nn_conv3x3", _p(x), B, H, W, cin, _p(w), cout, _p(bias), _p(y), _p(yb), 1, sp)
+    assert torch.equal(y, ye) and torch.equal(yb, yeb)
+    # data gradient: the k order of the flipped-weight GEMM, accumulated
+    wf, wt = (torch.empty(9 * cin * cout, dtype=torch.bfloat16, device="cuda") for _ in range(2))
+    nat.call("lbm_nn_conv3x3_flip_weights", _p(w), cin, cout, _p(wf), sp)
+    nat.call("lbm_nn_conv3x3_transpose_weights", _p(w), cin, cout, _p(wt), sp)
+    assert torch.equal(wt.view(cin, 9, cout), wf.view(9, cout, cin).permute(2, 0, 1))
+    dxe, dx = (torch.full((P, cin), 0.25, device="cuda") for _ in range(2))
+    nat.call("lbm_nn_conv3x3_dgrad", _p(dy), _p(wf), B, H, W, cin, cout, _p(dxe), 1, sp)
+    nat.call("lbm_nn_conv3x3_dgrad_t", _p(dy), _p(wt), B, H, W, cin, cout, _p(dx), 1, sp)
+    assert torch.equal(dx, dxe)
+    # weight gradient against float64: FP32 sums of exact products, at most P / 32
+    # MFMA steps of 32 products with one rounding each (bounded by 8 per step)
+    ref = (dy.view(P, cout).double().t() @ cols.double()).cpu()
+    bound = (dy.view(P, cout).double().abs().t() @ cols.double().abs()).cpu() * (P / 4) * 2.0 ** -24
+    for ks in (1, int(lib.lbm_nn_conv3x3_wgrad_splits(B, H, W, cin, cout))):
+        work = torch.empty(max(1, int(lib.lbm_nn_gemm_workspace(cout, K, ks)) // 4), device="cuda")
+        dw = torch.full((cout, K), float("nan"), device="cuda")
+        nat.call("lbm_nn_conv3x3_wgrad", _p(x), _p(dy), B, H, W, cin, cout, _p(dw), ks, _p(work), sp)
+        err = (dw.double().cpu() - ref).abs()
+        assert bool((err <= bound).all()), float((err / bound).max())
+        assert float(err.max()) < 1e-3 * float(ref.abs().max())
+    assert lib.lbm_nn_conv3x3_wgrad_splits(0, 1, 1, 1, 1) == -2
+    assert lib.lbm_nn_conv3x3_transpose_weights(None, cin, cout, _p(wt), sp) == -1
+    assert lib.lbm_nn_conv3x3_dgrad_t(None, _p(wt), B, H, W, cin, cout, _p(dx), 0, sp) == -1
