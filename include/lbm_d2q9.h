@@ -385,6 +385,11 @@ int lbm_nn_relu_backward(const float *y, float *dy, void *dy_bf16, int64_t n, vo
  * lbm_nn_bias_grad_workspace(N) bytes.                                       */
 int64_t lbm_nn_bias_grad_workspace(int N);
 int lbm_nn_bias_grad(const float *dy, int64_t M, int N, float *db, double *work, void *stream);
+/* A layer's backward before its GEMMs: dy_bf16 = BF16 of g, g = dy where y > 0
+ * (y NULL: g = dy), and db = column sums of g.  work as for lbm_nn_bias_grad;
+ * dy may be left holding dy or g.                                            */
+int lbm_nn_grad_epilogue(const float *y, float *dy, void *dy_bf16, int64_t M, int N, float *db,
+                         double *work, void *stream);
 /* 2x2 average pool x [B][H][W][C] -> y [B][H/2][W/2][C] (+ optional BF16 copy). */
 int lbm_nn_avgpool2(const float *x, int B, int H, int W, int C, float *y, void *yb, void *stream);
 int lbm_nn_avgpool2_backward(const float *dy, int B, int H, int W, int C, float *dx,

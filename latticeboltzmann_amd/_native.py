@@ -141,6 +141,7 @@ SIGNATURES = {
     "lbm_nn_relu_backward": (_i32, [_vp, _vp, _vp, _i64, _vp]),
     "lbm_nn_bias_grad_workspace": (_i64, [_i32]),
     "lbm_nn_bias_grad": (_i32, [_vp, _i64, _i32, _vp, _vp, _vp]),
+    "lbm_nn_grad_epilogue": (_i32, [_vp, _vp, _vp, _i64, _i32, _vp, _vp, _vp]),
     "lbm_nn_avgpool2": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp, _vp]),
     "lbm_nn_avgpool2_backward": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _i32, _vp]),
     "lbm_nn_upsample2": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp, _i32, _i32, _vp]),

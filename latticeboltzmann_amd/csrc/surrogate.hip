@@ -15,6 +15,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <initializer_list>
+
 #include "d2q9_node.hpp"
 #include "d2q9_reduce.hpp"
 #include "lbm_internal.hpp"
@@ -550,6 +552,28 @@ __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a) {
     }
 }
 
+// out = sum of k_wgrad's partials (splits x n values).  32 values a block and 8
+// threads a value, each adding every eighth partial in order: there are few
+// values and hundreds of partials, and one thread a value waits for one load
+// after another (28 us a layer; 64 partials took 13).
+__global__ __launch_bounds__(256) void k_wgrad_reduce(const float *__restrict__ work, int n, int splits,
+                                                      float *__restrict__ out) {
+    __shared__ float part[8][32];
+    const int e = threadIdx.x & 31, g = threadIdx.x >> 5;
+    const int i = blockIdx.x * 32 + e;
+    float v = 0.0f;
+    if (i < n) {
+#pragma unroll 4
+        for (int z = g; z < splits; z += 8) v += work[int64_t(z) * n + i];
+    }
+    part[g][e] = v;
+    __syncthreads();
+    if (g || i >= n) return;
+#pragma unroll
+    for (int q = 1; q < 8; ++q) v += part[q][e];
+    out[i] = v;
+}
+
 // im2col for 3x3 same convolution: x [B][H][W][C] BF16 -> cols [B*H*W][9*C].
 // Tap (dy, dx) = (blockIdx.y / 3, blockIdx.y % 3); each thread moves VEC
 // consecutive channels of one pixel (VEC = 8: one 16-byte load and store,
@@ -614,7 +638,7 @@ __global__ __launch_bounds__(256) void k_relu_backward(const float *__restrict__
 // rows [b*rows, (b+1)*rows) of columns [c0, c0 + cw), cw = min(N - c0, 256);
 // thread t owns column c0 + t % cw and rows t / cw, + 256 / cw, ... (coalesced
 // across a row), the threads of one column are then added in LDS in order.
-constexpr int kBiasBlocks = 256;
+constexpr int kBiasBlocks = 1024;
 
 __global__ __launch_bounds__(256) void k_bias_grad_partial(const float *__restrict__ dy, int64_t M,
                                                            int N, int c0, int64_t rows,
@@ -637,13 +661,59 @@ __global__ __launch_bounds__(256) void k_bias_grad_partial(const float *__restri
     }
 }
 
-// Pass 2: block n adds the nblocks (<= 256) partials of column n, one per
-// thread, in a fixed-shape tree, so all of them are loaded at once instead of
+// Pass 1 of a layer's backward epilogue: g = dy where y > 0 (y null: everywhere),
+// its BF16 copy, and the partial column sums of g in the same pass.  Four
+// columns a thread (N % 4 == 0): 16-byte loads, and enough of them in flight.
+// The masked FP32 gradient itself has no reader and is not written.
+__global__ __launch_bounds__(256) void k_grad_epilogue(const float *__restrict__ y, const float *__restrict__ dy,
+                                                       int64_t M, int N, int c0, int64_t rows,
+                                                       uint16_t *__restrict__ dyb,
+                                                       double *__restrict__ partial) {
+    __shared__ double red[4][256];
+    const int cw = min(N - c0, 256) / 4, t = threadIdx.x;  // column groups
+    const int lanes = 256 / cw, cg = t % cw, r0 = t / cw;
+    double s[4] = {0.0, 0.0, 0.0, 0.0};
+    if (r0 < lanes) {
+        const int64_t beg = int64_t(blockIdx.x) * rows, end = min(M, beg + rows);
+#pragma unroll 4
+        for (int64_t m = beg + r0; m < end; m += lanes) {
+            const int64_t o = m * N + c0 + cg * 4;
+            float4 g = *reinterpret_cast<const float4 *>(dy + o);
+            if (y) {
+                const float4 v = *reinterpret_cast<const float4 *>(y + o);
+                g.x = v.x > 0.0f ? g.x : 0.0f;
+                g.y = v.y > 0.0f ? g.y : 0.0f;
+                g.z = v.z > 0.0f ? g.z : 0.0f;
+                g.w = v.w > 0.0f ? g.w : 0.0f;
+            }
+            *reinterpret_cast<ushort4 *>(dyb + o) = make_ushort4(f2bf(g.x), f2bf(g.y), f2bf(g.z), f2bf(g.w));
+            s[0] += double(g.x);
+            s[1] += double(g.y);
+            s[2] += double(g.z);
+            s[3] += double(g.w);
+        }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) red[i][t] = s[i];
+    __syncthreads();
+    if (t < cw) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            double v = 0.0;
+            for (int j = 0; j < lanes; ++j) v += red[i][j * cw + t];
+            partial[int64_t(blockIdx.x) * N + c0 + t * 4 + i] = v;
+        }
+    }
+}
+
+// Pass 2: block n adds the nblocks partials of column n, one per thread at a
+// time, in a fixed-shape tree, so all of them are loaded at once instead of
 // one after another by a single thread.
 __global__ __launch_bounds__(256) void k_bias_grad_final(const double *__restrict__ partial, int N,
                                                          int nblocks, float *__restrict__ db) {
     const int n = blockIdx.x, t = threadIdx.x;
-    const double v = t < nblocks ? partial[int64_t(t) * N + n] : 0.0;
+    double v = 0.0;
+    for (int b = t; b < nblocks; b += 256) v += partial[int64_t(b) * N + n];
     const double tot = block_sum(v);
     if (t == 0) db[n] = float(tot);
 }
@@ -670,93 +740,136 @@ __global__ __launch_bounds__(256) void k_flip_weights(const uint16_t *__restrict
     wf[i] = w[(int64_t(co) * 9 + tap) * cin + c];
 }
 
+// V channels of one pixel: 4 (16-byte words) where the channel counts, offsets
+// and pointers allow it, else 1.  These kernels move memory and little else; with
+// one channel a thread they were bound by their index arithmetic (the network's
+// three upsamplings at batch 16: 27.5 us on average against 12.4; channel
+// copies 14.9 against 10.4, the pool's backward 15.3 against 7.4).
+template <int V>
+struct Vec {
+    float v[V];
+    __device__ __forceinline__ static Vec load(const float *p) {
+        Vec r;
+        if constexpr (V == 4) {
+            const float4 q = *reinterpret_cast<const float4 *>(p);
+            r.v[0] = q.x, r.v[1] = q.y, r.v[2] = q.z, r.v[3] = q.w;
+        } else {
+            r.v[0] = *p;
+        }
+        return r;
+    }
+    __device__ __forceinline__ void store(float *p) const {
+        if constexpr (V == 4) *reinterpret_cast<float4 *>(p) = make_float4(v[0], v[1], v[2], v[3]);
+        else *p = v[0];
+    }
+    __device__ __forceinline__ void store_bf16(uint16_t *p) const {
+        if constexpr (V == 4)
+            *reinterpret_cast<ushort4 *>(p) = make_ushort4(f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3]));
+        else *p = f2bf(v[0]);
+    }
+};
+
+// Pixel and channel of item idx of a [B][H][W][C] array taken V channels at a time.
+struct Pixel {
+    int c, x, y, b;
+    int64_t p;
+    __device__ __forceinline__ Pixel(int64_t idx, int cv, int V, int H, int W) {
+        c = int(idx % cv) * V;
+        p = idx / cv;
+        x = int(p % W);
+        const int64_t r = p / W;
+        y = int(r % H);
+        b = int(r / H);
+    }
+};
+
 // 2x2 average pool (NHWC): y [B][H/2][W/2][C].
+template <int V>
 __global__ __launch_bounds__(256) void k_avgpool2(const float *__restrict__ x, int B, int H, int W, int C,
                                                   float *__restrict__ y, uint16_t *__restrict__ yb) {
-    const int Ho = H / 2, Wo = W / 2;
     const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= int64_t(B) * Ho * Wo * C) return;
-    const int c = int(idx % C);
-    int64_t r = idx / C;
-    const int xo = int(r % Wo);
-    const int64_t r2 = r / Wo;
-    const int yo = int(r2 % Ho);
-    const int b = int(r2 / Ho);
-    const float *p = x + ((int64_t(b) * H + 2 * yo) * W + 2 * xo) * C + c;
-    const float v = 0.25f * ((p[0] + p[C]) + (p[int64_t(W) * C] + p[int64_t(W) * C + C]));
-    y[idx] = v;
-    if (yb) yb[idx] = f2bf(v);
+    if (idx >= int64_t(B) * (H / 2) * (W / 2) * (C / V)) return;
+    const Pixel o(idx, C / V, V, H / 2, W / 2);
+    const float *p = x + ((int64_t(o.b) * H + 2 * o.y) * W + 2 * o.x) * C + o.c;
+    const Vec<V> q0 = Vec<V>::load(p), q1 = Vec<V>::load(p + C);
+    const Vec<V> q2 = Vec<V>::load(p + int64_t(W) * C), q3 = Vec<V>::load(p + int64_t(W) * C + C);
+    Vec<V> r;
+#pragma unroll
+    for (int i = 0; i < V; ++i) r.v[i] = 0.25f * ((q0.v[i] + q1.v[i]) + (q2.v[i] + q3.v[i]));
+    r.store(y + idx * V);
+    if (yb) r.store_bf16(yb + idx * V);
 }
 
+template <int V>
 __global__ __launch_bounds__(256) void k_avgpool2_backward(const float *__restrict__ dy, int B, int H,
                                                            int W, int C, float *__restrict__ dx,
                                                            int accumulate) {
     const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= int64_t(B) * H * W * C) return;
-    const int c = int(idx % C);
-    int64_t r = idx / C;
-    const int xw = int(r % W);
-    const int64_t r2 = r / W;
-    const int yh = int(r2 % H);
-    const int b = int(r2 / H);
-    const float g = 0.25f * dy[((int64_t(b) * (H / 2) + yh / 2) * (W / 2) + xw / 2) * C + c];
-    dx[idx] = accumulate ? dx[idx] + g : g;
+    if (idx >= int64_t(B) * H * W * (C / V)) return;
+    const Pixel o(idx, C / V, V, H, W);
+    Vec<V> g = Vec<V>::load(dy + ((int64_t(o.b) * (H / 2) + o.y / 2) * (W / 2) + o.x / 2) * C + o.c);
+#pragma unroll
+    for (int i = 0; i < V; ++i) g.v[i] = 0.25f * g.v[i];
+    if (accumulate) {
+        const Vec<V> q = Vec<V>::load(dx + idx * V);
+#pragma unroll
+        for (int i = 0; i < V; ++i) g.v[i] = q.v[i] + g.v[i];
+    }
+    g.store(dx + idx * V);
 }
 
 // Nearest 2x upsample of x [B][H][W][C] into channels [coff, coff + C) of
 // y [B][2H][2W][Ct].
+template <int V>
 __global__ __launch_bounds__(256) void k_upsample2(const float *__restrict__ x, int B, int H, int W,
                                                    int C, float *__restrict__ y,
                                                    uint16_t *__restrict__ yb, int Ct, int coff) {
     const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    const int Ho = 2 * H, Wo = 2 * W;
-    if (idx >= int64_t(B) * Ho * Wo * C) return;
-    const int c = int(idx % C);
-    int64_t r = idx / C;  // output pixel
-    const int xo = int(r % Wo);
-    const int64_t r2 = r / Wo;
-    const int yo = int(r2 % Ho);
-    const int b = int(r2 / Ho);
-    const float v = x[((int64_t(b) * H + yo / 2) * W + xo / 2) * C + c];
-    const int64_t o = r * Ct + coff + c;
-    y[o] = v;
-    if (yb) yb[o] = f2bf(v);
+    if (idx >= int64_t(B) * 4 * H * W * (C / V)) return;
+    const Pixel o(idx, C / V, V, 2 * H, 2 * W);
+    const Vec<V> v = Vec<V>::load(x + ((int64_t(o.b) * H + o.y / 2) * W + o.x / 2) * C + o.c);
+    v.store(y + o.p * Ct + coff + o.c);
+    if (yb) v.store_bf16(yb + o.p * Ct + coff + o.c);
 }
 
+template <int V>
 __global__ __launch_bounds__(256) void k_upsample2_backward(const float *__restrict__ dy, int B, int H,
                                                             int W, int C, int Ct, int coff,
                                                             float *__restrict__ dx) {
     const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= int64_t(B) * H * W * C) return;
-    const int c = int(idx % C);
-    int64_t r = idx / C;
-    const int xw = int(r % W);
-    const int64_t r2 = r / W;
-    const int yh = int(r2 % H);
-    const int b = int(r2 / H);
-    const int Wo = 2 * W;
-    float s = 0.0f;
+    if (idx >= int64_t(B) * H * W * (C / V)) return;
+    const Pixel o(idx, C / V, V, H, W);
+    Vec<V> s;
+#pragma unroll
+    for (int i = 0; i < V; ++i) s.v[i] = 0.0f;
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
-        const int yo = 2 * yh + q / 2, xo = 2 * xw + q % 2;
-        s += dy[((int64_t(b) * (2 * H) + yo) * Wo + xo) * Ct + coff + c];
+        const int yo = 2 * o.y + q / 2, xo = 2 * o.x + q % 2;
+        const Vec<V> g = Vec<V>::load(dy + ((int64_t(o.b) * (2 * H) + yo) * (2 * W) + xo) * Ct + coff + o.c);
+#pragma unroll
+        for (int i = 0; i < V; ++i) s.v[i] += g.v[i];
     }
-    dx[idx] = s;
+    s.store(dx + idx * V);
 }
 
 // Channel-slice copy: dst[p][doff + c] (+)= src[p][soff + c] for c < C.
+template <int V>
 __global__ __launch_bounds__(256) void k_copy_channels(const float *__restrict__ src, int Cs, int soff,
                                                        float *__restrict__ dst, uint16_t *__restrict__ dstb,
                                                        int Cd, int doff, int C, int64_t P, int accumulate) {
     const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
-    if (idx >= P * C) return;
-    const int c = int(idx % C);
-    const int64_t p = idx / C;
-    float v = src[p * Cs + soff + c];
-    const int64_t o = p * Cd + doff + c;
-    if (accumulate) v += dst[o];
-    dst[o] = v;
-    if (dstb) dstb[o] = f2bf(v);
+    const int cv = C / V;
+    if (idx >= P * cv) return;
+    const int c = int(idx % cv) * V;
+    const int64_t p = idx / cv, o = p * Cd + doff + c;
+    Vec<V> v = Vec<V>::load(src + p * Cs + soff + c);
+    if (accumulate) {
+        const Vec<V> q = Vec<V>::load(dst + o);
+#pragma unroll
+        for (int i = 0; i < V; ++i) v.v[i] += q.v[i];
+    }
+    v.store(dst + o);
+    if (dstb) v.store_bf16(dstb + o);
 }
 
 // Mean squared error over n values: loss partials and dy = 2 (y - t) / n.
@@ -1021,6 +1134,16 @@ static int run_gemm(const GemmArgs &g, int splits, hipStream_t s) {
     return launch_status();
 }
 
+// Whether all counts are multiples of 4 and all pointers 16-byte aligned (8 for
+// the BF16 ones): Vec<4>.
+static bool by_four(std::initializer_list<int> counts, std::initializer_list<const void *> f32, const void *bf16) {
+    for (int c : counts)
+        if (c % 4) return false;
+    for (const void *q : f32)
+        if (reinterpret_cast<uintptr_t>(q) % 16) return false;
+    return reinterpret_cast<uintptr_t>(bf16) % 8 == 0;
+}
+
 // k_conv3 where it applies: C a multiple of the 32 channels of a step, 16-byte
 // aligned operands and (vector stores) outputs, operands below 2^31 bytes.
 static bool conv_direct(const ConvArgs &a) {
@@ -1133,9 +1256,8 @@ int lbm_nn_conv3x3_wgrad(const void *x, const void *dy, int B, int H, int W, int
         if (co == 64) hipLaunchKernelGGL(k_wgrad<4>, grid, dim3(256), 0, s, a);
         else hipLaunchKernelGGL(k_wgrad<2>, grid, dim3(256), 0, s, a);
         if (splits > 1) {
-            GemmArgs g{};
-            g.C = dw, g.ldc = N, g.M = cout, g.N = N, g.work = work;
-            hipLaunchKernelGGL(k_gemm_reduce, dim3(blocks_for(int64_t(cout) * N)), dim3(256), 0, s, g, splits);
+            hipLaunchKernelGGL(k_wgrad_reduce, dim3(blocks_for(int64_t(cout) * N, 32)), dim3(256), 0, s, work,
+                               cout * N, splits, dw);
         }
         return launch_status();
     }
@@ -1246,11 +1368,37 @@ int lbm_nn_bias_grad(const float *dy, int64_t M, int N, float *db, double *work,
     return launch_status();
 }
 
+int lbm_nn_grad_epilogue(const float *y, float *dy, void *dy_bf16, int64_t M, int N, float *db,
+                         double *work, void *stream) {
+    if (!dy || !dy_bf16 || !db || !work) return LBM_E_NULL;
+    if (M <= 0 || N <= 0) return LBM_E_SIZE;
+    hipStream_t s = as_stream(stream);
+    const bool vec = N % 4 == 0 && reinterpret_cast<uintptr_t>(y) % 16 == 0 &&
+                     reinterpret_cast<uintptr_t>(dy) % 16 == 0 && reinterpret_cast<uintptr_t>(dy_bf16) % 8 == 0;
+    if (!vec) {
+        const int rc = y ? lbm_nn_relu_backward(y, dy, dy_bf16, M * N, stream)
+                         : lbm_nn_to_bf16(dy, dy_bf16, M * N, stream);
+        return rc ? rc : lbm_nn_bias_grad(dy, M, N, db, work, stream);
+    }
+    const int64_t rows = (M + kBiasBlocks - 1) / kBiasBlocks;
+    const int nb = int((M + rows - 1) / rows);
+    for (int c0 = 0; c0 < N; c0 += 256)
+        hipLaunchKernelGGL(k_grad_epilogue, dim3(nb), dim3(256), 0, s, y, dy, M, N, c0, rows,
+                           static_cast<uint16_t *>(dy_bf16), work);
+    hipLaunchKernelGGL(k_bias_grad_final, dim3(N), dim3(256), 0, s, work, N, nb, db);
+    return launch_status();
+}
+
 int lbm_nn_avgpool2(const float *x, int B, int H, int W, int C, float *y, void *yb, void *stream) {
     if (!x || !y) return LBM_E_NULL;
     if (B <= 0 || H < 2 || W < 2 || C <= 0 || (H & 1) || (W & 1)) return LBM_E_SIZE;
-    hipLaunchKernelGGL(k_avgpool2, dim3(blocks_for(int64_t(B) * (H / 2) * (W / 2) * C)), dim3(256), 0,
-                       as_stream(stream), x, B, H, W, C, y, static_cast<uint16_t *>(yb));
+    const int64_t n = int64_t(B) * (H / 2) * (W / 2) * C;
+    if (by_four({C}, {x, y}, yb))
+        hipLaunchKernelGGL(k_avgpool2<4>, dim3(blocks_for(n / 4)), dim3(256), 0, as_stream(stream), x, B, H, W,
+                           C, y, static_cast<uint16_t *>(yb));
+    else
+        hipLaunchKernelGGL(k_avgpool2<1>, dim3(blocks_for(n)), dim3(256), 0, as_stream(stream), x, B, H, W, C,
+                           y, static_cast<uint16_t *>(yb));
     return launch_status();
 }
 
@@ -1258,8 +1406,13 @@ int lbm_nn_avgpool2_backward(const float *dy, int B, int H, int W, int C, float 
                              void *stream) {
     if (!dy || !dx) return LBM_E_NULL;
     if (B <= 0 || H < 2 || W < 2 || C <= 0 || (H & 1) || (W & 1)) return LBM_E_SIZE;
-    hipLaunchKernelGGL(k_avgpool2_backward, dim3(blocks_for(int64_t(B) * H * W * C)), dim3(256), 0,
-                       as_stream(stream), dy, B, H, W, C, dx, accumulate);
+    const int64_t n = int64_t(B) * H * W * C;
+    if (by_four({C}, {dy, dx}, nullptr))
+        hipLaunchKernelGGL(k_avgpool2_backward<4>, dim3(blocks_for(n / 4)), dim3(256), 0, as_stream(stream), dy,
+                           B, H, W, C, dx, accumulate);
+    else
+        hipLaunchKernelGGL(k_avgpool2_backward<1>, dim3(blocks_for(n)), dim3(256), 0, as_stream(stream), dy, B,
+                           H, W, C, dx, accumulate);
     return launch_status();
 }
 
@@ -1267,8 +1420,13 @@ int lbm_nn_upsample2(const float *x, int B, int H, int W, int C, float *y, void 
                      void *stream) {
     if (!x || !y) return LBM_E_NULL;
     if (B <= 0 || H <= 0 || W <= 0 || C <= 0 || coff < 0 || coff + C > Ct) return LBM_E_SIZE;
-    hipLaunchKernelGGL(k_upsample2, dim3(blocks_for(int64_t(B) * 4 * H * W * C)), dim3(256), 0,
-                       as_stream(stream), x, B, H, W, C, y, static_cast<uint16_t *>(yb), Ct, coff);
+    const int64_t n = int64_t(B) * 4 * H * W * C;
+    if (by_four({C, Ct, coff}, {x, y}, yb))
+        hipLaunchKernelGGL(k_upsample2<4>, dim3(blocks_for(n / 4)), dim3(256), 0, as_stream(stream), x, B, H, W,
+                           C, y, static_cast<uint16_t *>(yb), Ct, coff);
+    else
+        hipLaunchKernelGGL(k_upsample2<1>, dim3(blocks_for(n)), dim3(256), 0, as_stream(stream), x, B, H, W, C,
+                           y, static_cast<uint16_t *>(yb), Ct, coff);
     return launch_status();
 }
 
@@ -1276,8 +1434,13 @@ int lbm_nn_upsample2_backward(const float *dy, int B, int H, int W, int C, int C
                               float *dx, void *stream) {
     if (!dy || !dx) return LBM_E_NULL;
     if (B <= 0 || H <= 0 || W <= 0 || C <= 0 || coff < 0 || coff + C > Ct) return LBM_E_SIZE;
-    hipLaunchKernelGGL(k_upsample2_backward, dim3(blocks_for(int64_t(B) * H * W * C)), dim3(256), 0,
-                       as_stream(stream), dy, B, H, W, C, Ct, coff, dx);
+    const int64_t n = int64_t(B) * H * W * C;
+    if (by_four({C, Ct, coff}, {dy, dx}, nullptr))
+        hipLaunchKernelGGL(k_upsample2_backward<4>, dim3(blocks_for(n / 4)), dim3(256), 0, as_stream(stream),
+                           dy, B, H, W, C, Ct, coff, dx);
+    else
+        hipLaunchKernelGGL(k_upsample2_backward<1>, dim3(blocks_for(n)), dim3(256), 0, as_stream(stream), dy, B,
+                           H, W, C, Ct, coff, dx);
     return launch_status();
 }
 
@@ -1285,8 +1448,12 @@ int lbm_nn_copy_channels(const float *src, int Cs, int soff, float *dst, void *d
                          int doff, int C, int64_t P, int accumulate, void *stream) {
     if (!src || !dst) return LBM_E_NULL;
     if (C <= 0 || P <= 0 || soff < 0 || doff < 0 || soff + C > Cs || doff + C > Cd) return LBM_E_SIZE;
-    hipLaunchKernelGGL(k_copy_channels, dim3(blocks_for(P * C)), dim3(256), 0, as_stream(stream), src,
-                       Cs, soff, dst, static_cast<uint16_t *>(dst_bf16), Cd, doff, C, P, accumulate);
+    if (by_four({C, Cs, soff, Cd, doff}, {src, dst}, dst_bf16))
+        hipLaunchKernelGGL(k_copy_channels<4>, dim3(blocks_for(P * C / 4)), dim3(256), 0, as_stream(stream),
+                           src, Cs, soff, dst, static_cast<uint16_t *>(dst_bf16), Cd, doff, C, P, accumulate);
+    else
+        hipLaunchKernelGGL(k_copy_channels<1>, dim3(blocks_for(P * C)), dim3(256), 0, as_stream(stream), src, Cs,
+                           soff, dst, static_cast<uint16_t *>(dst_bf16), Cd, doff, C, P, accumulate);
     return launch_status();
 }
 

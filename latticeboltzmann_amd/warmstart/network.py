@@ -183,11 +183,11 @@ class Surrogate:
         s = nat.stream_ptr()
         dy = dy.contiguous()
         dyb = torch.empty_like(dy, dtype=torch.bfloat16)
-        if relu:
-            nat.call("lbm_nn_relu_backward", _p(y), _p(dy), _p(dyb), dy.numel(), s)
-        else:
-            nat.call("lbm_nn_to_bf16", _p(dy), _p(dyb), dy.numel(), s)
         gw, gbias = self.views(name, self.g)
+        bw = torch.empty(int(nat.load().lbm_nn_bias_grad_workspace(cout)) // 8, dtype=torch.float64,
+                         device=self.device)
+        nat.call("lbm_nn_grad_epilogue", _p(y) if relu else None, _p(dy), _p(dyb), P, cout, _p(gbias),
+                 _p(bw), s)
         ks = int(nat.load().lbm_nn_conv3x3_wgrad_splits(B, H, W, cin, cout))
         work = None
         if ks > 1:
@@ -196,9 +196,6 @@ class Surrogate:
         # dW[co][k] = sum_p dy[p][co] x(p, k), x(p, k) the gathered 3x3 neighbourhood
         nat.call("lbm_nn_conv3x3_wgrad", _p(xb), _p(dyb), B, H, W, cin, cout, _p(gw), ks,
                  None if work is None else _p(work), s)
-        bw = torch.empty(int(nat.load().lbm_nn_bias_grad_workspace(cout)) // 8, dtype=torch.float64,
-                         device=self.device)
-        nat.call("lbm_nn_bias_grad", _p(dy), P, cout, _p(gbias), _p(bw), s)
         if not need_dx:
             return None
         # dx[p][c] = sum over taps and co of dy[p - tap][co] W[co][tap][c]
