@@ -87,7 +87,7 @@ int lbm_moments_f32(const float *f, int64_t nx, int64_t ny, int layout, float *r
 int lbm_stream_periodic(const void *src, void *dst, int64_t nx, int64_t ny,
                         int elem_bytes, void *stream);
 
-/* K full time steps src -> dst in one launch (temporal blocking, K = 2..6
+/* K full time steps src -> dst in one launch (temporal blocking, K = 2..8
  * fixed by the variant).  Tile variants: each block computes the first K-1
  * steps of its tile and a shrinking halo in LDS and writes only the last.
  * Sweep variants: each wave walks a strip of 64 columns along x and keeps the
@@ -107,9 +107,9 @@ int lbm_step_multi_f32(const float *src, float *dst, int64_t nx, int64_t ny, int
                        int variant, void *stream);
 int lbm_step_multi_variant_count(void);
 int lbm_step_multi_default_variant(void); /* the FP64 tile default (below 4096^2 nodes) */
-/* The variant that -1 selects on an nx x ny grid: the default tile below
- * 4096^2 nodes, the five-step register sweep from there (LBM_E_SIZE for an
- * invalid grid); _f32 for lbm_step_multi_f32, whose tile default differs.
+/* The variant that -1 selects on an nx x ny grid: small tiles for grids of
+ * few default tiles, the default tile below 4096^2 nodes, the five-step register
+ * sweep from there (LBM_E_SIZE for an invalid grid); _f32 for lbm_step_multi_f32, whose tile default differs.
  * No counterpart in the reference (its driver steps one step per call).       */
 int lbm_step_multi_default_for(int64_t nx, int64_t ny);
 int lbm_step_multi_default_for_f32(int64_t nx, int64_t ny);

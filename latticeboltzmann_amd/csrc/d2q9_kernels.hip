@@ -107,7 +107,7 @@ __global__ __launch_bounds__(BS) void k_step(const T *__restrict__ src, T *__res
     }
 }
 
-// K fused steps per launch (temporal blocking, K = 2..4), src -> dst.
+// K fused steps per launch (temporal blocking, K = 2..8), src -> dst.
 // Block b owns a TR x TC tile of nodes.  Phase 1 computes step 1 on the tile
 // and a halo ring K-1 nodes deep, at wrapped global coordinates, with the
 // single-step node code (pull from src, walls, collide), into LDS; each later
@@ -205,6 +205,17 @@ __device__ __forceinline__ void phase_lds(T *buf, int k0, int l0, int nx, int ny
     }
 }
 
+// The LDS phases of halo H, H - 1, ..., 1.
+template <typename T, int BC, int TR, int TC, int H, int BS>
+__device__ __forceinline__ void lds_phases(T *buf, int k0, int l0, int nx, int ny, T omega, T u0,
+                                           bool edge) {
+    if constexpr (H >= 1) {
+        phase_lds<T, BC, TR, TC, H, BS>(buf, k0, l0, nx, ny, omega, u0, edge);
+        __syncthreads();
+        lds_phases<T, BC, TR, TC, H - 1, BS>(buf, k0, l0, nx, ny, omega, u0, edge);
+    }
+}
+
 // Last phase: the tile from halo-1 LDS values to dst.
 template <typename T, int BC, bool MOM, int TR, int TC, int BS, bool NTS>
 __device__ __forceinline__ void phase_to_global(const T *in, T *__restrict__ dst, int k0, int l0,
@@ -240,7 +251,7 @@ __global__ __launch_bounds__(BS) void k_stepk(const T *__restrict__ src, T *__re
                                                   int nx, int ny, Layout L, int ntc, int ntiles,
                                                   T omega, T u0, T *__restrict__ rho_o,
                                                   T *__restrict__ ux_o, T *__restrict__ uy_o) {
-    static_assert(K >= 2 && K <= 4, "2 to 4 steps per launch");
+    static_assert(K >= 2 && K <= 8, "2 to 8 steps per launch");
     constexpr int NA = (TR + 2 * (K - 1)) * (TC + 2 * (K - 1));  // the phase-1 ring, the largest
     __shared__ T sa[9 * NA];
     const int tile = xcd_tile(ntiles);
@@ -255,14 +266,7 @@ __global__ __launch_bounds__(BS) void k_stepk(const T *__restrict__ src, T *__re
 
     phase_from_global<T, BC, TR, TC, K - 1, BS>(src, sa, k0, l0, nx, ny, L, omega, u0, edge);
     __syncthreads();
-    if constexpr (K >= 4) {
-        phase_lds<T, BC, TR, TC, 2, BS>(sa, k0, l0, nx, ny, omega, u0, edge);
-        __syncthreads();
-    }
-    if constexpr (K >= 3) {
-        phase_lds<T, BC, TR, TC, 1, BS>(sa, k0, l0, nx, ny, omega, u0, edge);
-        __syncthreads();
-    }
+    lds_phases<T, BC, TR, TC, K - 2, BS>(sa, k0, l0, nx, ny, omega, u0, edge);
     phase_to_global<T, BC, MOM, TR, TC, BS, NTS>(sa, dst, k0, l0, nx, ny, L, omega, u0, rho_o, ux_o, uy_o,
                                             edge);
 }
@@ -802,7 +806,23 @@ constexpr int kNumTileShapes = 0 LBM_MULTI_SHAPES(LBM_COUNT_MULTI);
     X(12, 5, 0, true, false, true)
 #define LBM_COUNT_SWEEP(id, k, seg, pp, pf, nts) +1
 constexpr int kNumSweepShapes = 0 LBM_SWEEP_SHAPES(LBM_COUNT_SWEEP);
-constexpr int kNumMultiShapes = kNumTileShapes + kNumSweepShapes;
+
+// Tile shapes for small grids (k_stepk; columns as LBM_MULTI_SHAPES), variants
+// after the sweeps.  Such a grid is a few blocks, each a serial chain of one
+// phase per step (about 1 us a phase and 3 us a launch), so a ring wants at most
+// one node per thread, and the tiles want to spread over all CUs.  us per step
+// in a replayed graph, against 8 x 32 / 512 threads and 22 x 32 / 768: FP64
+// 64^2 1.25 (8 x 8, K = 4) against 1.71 and 2.45; 256^2 1.71 (16 x 16, K = 4) and
+// 1.62 (K = 6) against 1.87 and 2.56.  Not kept: K = 5 on 16 x 16 (1.66 at
+// 256^2), K = 6 and 8 on 8 x 8 (1.18 and 1.16 at 64^2, but more single steps
+// left over), 8 x 16 and 4 x 16 tiles.
+#define LBM_SMALL_SHAPES(X)              \
+    X(0, 4, 16, 16, 512, false)      \
+    X(1, 6, 16, 16, 768, false)      \
+    X(2, 4, 8, 8, 256, false)
+constexpr int kFirstSmallShape = kNumTileShapes + kNumSweepShapes;
+constexpr int kNumSmallShapes = 0 LBM_SMALL_SHAPES(LBM_COUNT_MULTI);
+constexpr int kNumMultiShapes = kFirstSmallShape + kNumSmallShapes;
 // Four steps on 22 x 32 tiles with 768 threads: the fastest FP64 shape measured
 // (115 GLUPS at 2048^2, 120 at 3072^2, 124.5 at 4096^2, against 105-113, 113-115
 // and 120 for 20 x 32 tiles of 512 threads in the same runs).  76.6 KB of LDS,
@@ -830,7 +850,18 @@ constexpr int kDefaultMultiShapeF32 = 18;
 template <typename T>
 inline int default_multi_shape(int64_t nx, int64_t ny) {
     if (nx * ny >= kLargeGridNodes) return kLargeGridMultiShape;
-    return sizeof(T) == sizeof(float) ? kDefaultMultiShapeF32 : kDefaultMultiShape;
+    // Four steps a launch: six gain little (256^2: 1.62 us a step against 1.71) and
+    // leave up to five single steps.  8 x 8 tiles while each has a CU of its own
+    // (128^2: 1.28 us against 1.59 on 16 x 16 and 2.48 on 22 x 32); 16 x 16 while
+    // 22 x 32 tiles would leave half of the CUs idle (256^2: 1.71 against 2.56; at
+    // 384^2, 216 tiles of 22 x 32, they lose 2.75 to 2.55).
+    constexpr bool f32 = sizeof(T) == sizeof(float);
+    const int64_t cus = device_cus();
+    if (nx >= (f32 ? 28 : 30) && ny >= 40) {  // grids that the tile default takes
+        if (((nx + 7) / 8) * ((ny + 7) / 8) <= cus) return kFirstSmallShape + 2;
+        if (((nx + 21) / 22) * ((ny + 31) / 32) <= cus / 2) return kFirstSmallShape;
+    }
+    return f32 ? kDefaultMultiShapeF32 : kDefaultMultiShape;
 }
 
 template <typename T, int BC, bool MOM, int K, int TR, int TC, int BS, bool NTS>
@@ -874,13 +905,17 @@ int launch_multi_bc(const T *src, T *dst, int64_t nx, int64_t ny, Layout L, T om
                     T *ux, T *uy, int shape, hipStream_t s) {
 #define LBM_LAUNCH_MULTI(id, k, tr, tc, bs, nts) \
     case id: return launch_multi_v<T, BC, MOM, k, tr, tc, bs, nts>(src, dst, nx, ny, L, omega, u0, rho, ux, uy, s);
+#define LBM_LAUNCH_SMALL(id, k, tr, tc, bs, nts) \
+    case kFirstSmallShape + id: return launch_multi_v<T, BC, MOM, k, tr, tc, bs, nts>(src, dst, nx, ny, L, omega, u0, rho, ux, uy, s);
 #define LBM_LAUNCH_SWEEP(id, k, seg, pp, pf, nts) \
     case kNumTileShapes + id: return launch_sweep_v<T, BC, MOM, k, pp, pf, nts>(src, dst, nx, ny, L, seg, omega, u0, rho, ux, uy, s);
     switch (shape) {
         LBM_MULTI_SHAPES(LBM_LAUNCH_MULTI)
         LBM_SWEEP_SHAPES(LBM_LAUNCH_SWEEP)
+        LBM_SMALL_SHAPES(LBM_LAUNCH_SMALL)
         default: return LBM_E_ARG;
     }
+#undef LBM_LAUNCH_SMALL
 #undef LBM_LAUNCH_MULTI
 #undef LBM_LAUNCH_SWEEP
 }
@@ -914,13 +949,17 @@ inline int multi_shape_info(int variant, int *steps, int64_t *min_nx, int64_t *m
     const int shape = variant < 0 ? kDefaultMultiShape : variant;
 #define LBM_INFO_MULTI(id, k, tr, tc, bs, nts) \
     case id: *steps = k; *min_nx = tr + 2 * k; *min_ny = tc + 2 * k; return LBM_OK;
+#define LBM_INFO_SMALL(id, k, tr, tc, bs, nts) \
+    case kFirstSmallShape + id: *steps = k; *min_nx = tr + 2 * k; *min_ny = tc + 2 * k; return LBM_OK;
 #define LBM_INFO_SWEEP(id, k, seg, pp, pf, nts) \
     case kNumTileShapes + id: *steps = k; *min_nx = 2 * k; *min_ny = 64; return LBM_OK;
     switch (shape) {
         LBM_MULTI_SHAPES(LBM_INFO_MULTI)
         LBM_SWEEP_SHAPES(LBM_INFO_SWEEP)
+        LBM_SMALL_SHAPES(LBM_INFO_SMALL)
         default: return LBM_E_ARG;
     }
+#undef LBM_INFO_SMALL
 #undef LBM_INFO_MULTI
 #undef LBM_INFO_SWEEP
 }

@@ -49,7 +49,7 @@ class Lattice:
         autotuned; "auto" also tunes the multi-step kernel's shape).
     layout : ``"rows"`` (default) or ``"soa"`` (the reference's f[i][k][l]).
     multi_step : advance runs of K steps with the temporally blocked
-        multi-step kernel (``lbm_step_multi_*``, K = 2..4 per launch, bitwise
+        multi-step kernel (``lbm_step_multi_*``, K = 2..8 per launch, bitwise
         equal to K single steps) where the grid is large enough for its tiles.
     """
 

@@ -171,3 +171,22 @@ def test_step_graph_replay_after_odd_eager_steps(gpu):
     ref.step(8 + 1 + 8 + 3 + 8)
     assert lat.time == ref.time == 28
     assert np.array_equal(lat.populations(), ref.populations())
+
+
+@pytest.mark.parametrize("dtype", [torch.float64, torch.float32])
+@pytest.mark.parametrize("nx,ny", [(30, 40), (64, 64), (128, 128), (129, 128), (233, 257), (256, 352)])
+def test_small_grid_defaults_equal_single_steps(gpu, dtype, nx, ny):
+    # the default shapes of small grids, their remainders, and the moments of
+    # the last launch whichever kind it is
+    from latticeboltzmann_amd.lattice import Lattice
+    f = populations(nx, ny, dtype)
+    one = Lattice(nx, ny, 1.3, "cavity", 0.1, dtype, multi_step=False).load(f)
+    for n in (8, 13, 4, 17):
+        lat = Lattice(nx, ny, 1.3, "cavity", 0.1, dtype).load(f)
+        print("small", dtype, nx, ny, n, lat.multi_variant, lat.launches(n), flush=True)
+        one.load(f)
+        m, m1 = ([torch.empty((nx, ny), dtype=dtype, device="cuda") for _ in range(3)] for _ in range(2))
+        lat.step(n, moments=m)
+        one.step(n, moments=m1)
+        assert torch.equal(lat.f, one.f)
+        assert all(torch.equal(a, b) for a, b in zip(m, m1))
