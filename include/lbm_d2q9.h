@@ -87,6 +87,16 @@ int lbm_moments_f32(const float *f, int64_t nx, int64_t ny, int layout, float *r
 int lbm_stream_periodic(const void *src, void *dst, int64_t nx, int64_t ny,
                         int elem_bytes, void *stream);
 
+/* The same in place on f[9][nx][ny] (PyLB.stream modifies its argument).  scratch:
+ * lbm_stream_inplace_scratch(nx, ny, walls) elements of f's type, walls = 1 for the
+ * cavity form; it must not overlap f.  Element sizes 1, 2, 4 and 8.           */
+int64_t lbm_stream_inplace_scratch(int64_t nx, int64_t ny, int walls);
+int lbm_stream_inplace(void *f, int64_t nx, int64_t ny, int elem_bytes, void *scratch, void *stream);
+int lbm_stream_bounce_back_inplace_f64(double *f, int64_t nx, int64_t ny, double u0, double *scratch,
+                                       void *stream);
+int lbm_stream_bounce_back_inplace_f32(float *f, int64_t nx, int64_t ny, float u0, float *scratch,
+                                       void *stream);
+
 /* K full time steps src -> dst in one launch (temporal blocking, K = 2..8
  * fixed by the variant).  Tile variants: each block computes the first K-1
  * steps of its tile and a shrinking halo in LDS and writes only the last.

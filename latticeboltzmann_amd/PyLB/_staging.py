@@ -39,3 +39,9 @@ def write_back(dst, t):
     if host.dtype != dst.dtype:
         host = host.view(dst.dtype)
     dst[...] = host.reshape(dst.shape)
+
+
+def written(t):
+    """Tell autograd that the kernels have written tensor ``t`` in place."""
+    if not t.is_inference():
+        torch.autograd.graph.increment_version(t)

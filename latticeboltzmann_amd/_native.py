@@ -80,6 +80,10 @@ SIGNATURES = {
     "lbm_stream_periodic": (_i32, [_vp, _vp, _i64, _i64, _i32, _vp]),
     "lbm_stream_bounce_back_f64": (_i32, [_vp, _vp, _i64, _i64, _f64, _vp]),
     "lbm_stream_bounce_back_f32": (_i32, [_vp, _vp, _i64, _i64, _f32, _vp]),
+    "lbm_stream_inplace_scratch": (_i64, [_i64, _i64, _i32]),
+    "lbm_stream_inplace": (_i32, [_vp, _i64, _i64, _i32, _vp, _vp]),
+    "lbm_stream_bounce_back_inplace_f64": (_i32, [_vp, _i64, _i64, _f64, _vp, _vp]),
+    "lbm_stream_bounce_back_inplace_f32": (_i32, [_vp, _i64, _i64, _f32, _vp, _vp]),
     "lbm_step_f64": (_i32, [_vp, _vp, _i64, _i64, _f64, _i32, _f64, _vp, _vp, _vp, _i32, _vp]),
     "lbm_step_f32": (_i32, [_vp, _vp, _i64, _i64, _f32, _i32, _f32, _vp, _vp, _vp, _i32, _vp]),
     "lbm_step_layout_f64": (_i32, [_vp, _vp, _i64, _i64, _i32, _f64, _i32, _f64, _vp, _vp, _vp,

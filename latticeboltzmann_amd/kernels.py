@@ -145,6 +145,21 @@ def stream_bounce_back(f, u0=0.1, out=None):
     return out
 
 
+def stream_in_place(f, u0=None):
+    """``stream`` (u0 None) or ``stream_bounce_back`` of ``f`` in place."""
+    nx, ny = _populations(f, "stream")
+    n = int(nat.load().lbm_stream_inplace_scratch(nx, ny, int(u0 is not None)))
+    nat.check(min(n, 0), "lbm_stream_inplace_scratch")
+    scratch = torch.empty(n, dtype=f.dtype, device=f.device)
+    if u0 is None:
+        nat.call("lbm_stream_inplace", nat.ptr(f), nx, ny, f.element_size(), nat.ptr(scratch),
+                 nat.stream_ptr())
+    else:
+        nat.call("lbm_stream_bounce_back_inplace_" + _suffix(f, "stream_and_bounce_back"), nat.ptr(f),
+                 nx, ny, float(u0), nat.ptr(scratch), nat.stream_ptr())
+    return f
+
+
 def step(src, dst, omega, bc=nat.BC_CAVITY, u0=0.1, moments=None, variant=-1,
          layout=nat.LAYOUT_SOA):
     """One fused step ``src -> dst`` (pull streaming, walls if cavity, collide).

@@ -317,3 +317,45 @@ def test_copy_kernel(gpu):
     assert lib.lbm_copy(a.data_ptr(), b.data_ptr(), 8 * 9999, 0, s_) == -2        # not a multiple of 16
     assert lib.lbm_copy(a.data_ptr() + 8, b.data_ptr(), 16, 0, s_) == -3          # misaligned
     assert lib.lbm_copy(a.data_ptr(), a.data_ptr() + 16, 64, 0, s_) == -4         # overlap
+
+
+@pytest.mark.parametrize("nx,ny", [(1, 1), (1, 7), (7, 1), (2, 2), (3, 5), (16, 16), (17, 33), (32, 257),
+                                   (33, 300), (40, 2049), (5, 4101), (1000, 130),
+                                   (1153, 1021)])
+def test_streaming_in_place_equals_second_array(gpu, nx, ny):
+    # bands of 16 rows (whole, cut, one), rows longer than one chunk, chains that
+    # wrap several times within a band; walls on every degenerate grid
+    from latticeboltzmann_amd import PyLB, kernels
+    gen = torch.Generator(device="cuda").manual_seed(nx * 7 + ny)
+    for dt in (torch.uint8, torch.int16, torch.float32, torch.float64):
+        f = torch.randint(0, 250, (9, nx, ny), device="cuda", generator=gen).to(dt)
+        ref = kernels.stream(f)
+        got = f.clone()
+        PyLB.stream(got)
+        assert torch.equal(got, ref), dt
+    for dt in (torch.float32, torch.float64):
+        f = torch.rand((9, nx, ny), device="cuda", generator=gen, dtype=dt)
+        ref = kernels.stream_bounce_back(f, 0.07)
+        got = f.clone()
+        kernels.stream_in_place(got, 0.07)  # the kernel at any size
+        assert torch.equal(got, ref), dt
+        got = f.clone()
+        version = got._version
+        PyLB.stream_and_bounce_back(got, 0.07)
+        assert torch.equal(got, ref), dt
+        assert got._version > version
+    # other forms of the argument: a view with strides, a view at an odd offset,
+    # an autograd leaf (refused by copy_)
+    f = torch.rand((9, ny, nx), device="cuda", generator=gen, dtype=torch.float64)
+    t = f.transpose(1, 2)
+    ref = kernels.stream(t.contiguous())
+    PyLB.stream(t)
+    assert torch.equal(t, ref)
+    base = torch.rand(9 * nx * ny + 1, device="cuda", generator=gen)
+    v = base[1:].view(9, nx, ny)
+    ref, head = kernels.stream_bounce_back(v.clone(), 0.07), base[0].clone()
+    PyLB.stream_and_bounce_back(v, 0.07)
+    assert torch.equal(v, ref) and base[0] == head
+    leaf = torch.rand((9, nx, ny), device="cuda", requires_grad=True)
+    with pytest.raises(RuntimeError):
+        PyLB.stream(leaf)
