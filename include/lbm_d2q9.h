@@ -379,6 +379,33 @@ int lbm_nn_conv3x3_wgrad(const void *x, const void *dy, int B, int H, int W, int
 int lbm_nn_conv3x3_flip_weights(const void *w, int cin, int cout, void *wf, void *stream);
 int lbm_nn_conv3x3_dgrad(const void *dy, const void *wf, int B, int H, int W, int cin, int cout,
                          float *dx, int accumulate, void *stream);
+/* A network's convolutions with its weights packed in the order in which the MFMA
+ * fragments are loaded: lbm_nn_pack_weights packs the BF16 weights of n layers
+ * (element offsets from[] into w, to[] into out, multiples of 8; packed size of a
+ * layer: lbm_nn_packed_size) in one launch, for the forward pass or (transposed)
+ * the data gradient; layers whose cin (transposed: cout) is no multiple of 32 are
+ * left out.  conv3x3_packed takes both forms of the weights and the packed one
+ * (wp, nullable) where it applies; dgrad_packed returns LBM_E_ARG where it does
+ * not.  Results are the bits of conv3x3 and dgrad.                           */
+#define LBM_NN_MAX_LAYERS 32
+int64_t lbm_nn_packed_size(int cin, int cout);
+int lbm_nn_packed_fits(int B, int H, int W, int cin, int cout); /* 1 or 0 */
+int lbm_nn_pack_weights(const void *w, const int64_t *from, const int *cin, const int *cout, int n,
+                        int transposed, void *out, const int64_t *to, void *stream);
+int lbm_nn_conv3x3_packed(const void *x, int B, int H, int W, int cin, const void *w, const void *wp, int cout,
+                          const float *bias, float *y, void *yb, int relu, void *stream);
+/* One prediction of the U-Net, x (B, H, W, in_ch) FP32 -> out (B, H, W, out_ch):
+ * per level two ReLU convolutions and an average pool, two convolutions of mid
+ * channels, per level an upsample, the concatenation with the level's skip and
+ * two convolutions, a linear head.  p, pb: the layers' parameters, one after
+ * another as weights [cout][tap][cin] and bias, FP32 (biases) and BF16 (weights).
+ * work: lbm_nn_unet_workspace bytes, 16-byte aligned.  H, W multiples of
+ * 2^levels, levels <= 7.                                                      */
+int64_t lbm_nn_unet_workspace(int B, int H, int W, int in_ch, const int *widths, int levels, int mid, int out_ch);
+int lbm_nn_unet_forward(const float *x, int B, int H, int W, int in_ch, const int *widths, int levels, int mid,
+                        int out_ch, const float *p, const void *pb, void *work, float *out, void *stream);
+int lbm_nn_conv3x3_dgrad_packed(const void *dy, const void *wp, int B, int H, int W, int cin, int cout,
+                                float *dx, void *stream);
 /* The same from weights in wt[cin][tap][cout] (lbm_nn_conv3x3_transpose_weights):
  * k contiguous, which the direct kernel (cout a multiple of 32) loads as it is. */
 int lbm_nn_conv3x3_transpose_weights(const void *w, int cin, int cout, void *wt, void *stream);

@@ -37,6 +37,7 @@ _f64, _f32 = ctypes.c_double, ctypes.c_float
 
 RULE_COPY, RULE_LID, RULE_LID_RHO, RULE_ZERO = 0, 1, 2, 3
 GHOST_MAX_RULES = 32
+NN_MAX_LAYERS = 32
 PBC_NONE, PBC_BEFORE_STREAM, PBC_AFTER_STREAM = 0, 1, 2
 GHOST_NO_COLLIDE, GHOST_COLLIDE_ONLY = 1, 2
 
@@ -140,6 +141,14 @@ SIGNATURES = {
     "lbm_nn_conv3x3_dgrad": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _i32, _vp]),
     "lbm_nn_conv3x3_transpose_weights": (_i32, [_vp, _i32, _i32, _vp, _vp]),
     "lbm_nn_conv3x3_dgrad_t": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _i32, _vp]),
+    "lbm_nn_packed_fits": (_i32, [_i32, _i32, _i32, _i32, _i32]),
+    "lbm_nn_unet_workspace": (_i64, [_i32, _i32, _i32, _i32, _vp, _i32, _i32, _i32]),
+    "lbm_nn_unet_forward": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _i32, _i32, _i32, _vp, _vp, _vp, _vp,
+                                   _vp]),
+    "lbm_nn_packed_size": (_i64, [_i32, _i32]),
+    "lbm_nn_pack_weights": (_i32, [_vp, _vp, _vp, _vp, _i32, _i32, _vp, _vp, _vp]),
+    "lbm_nn_conv3x3_packed": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp, _i32, _vp, _vp, _vp, _i32, _vp]),
+    "lbm_nn_conv3x3_dgrad_packed": (_i32, [_vp, _vp, _i32, _i32, _i32, _i32, _i32, _vp, _vp]),
     "lbm_nn_im2col3x3": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _vp]),
     "lbm_nn_col2im3x3": (_i32, [_vp, _i32, _i32, _i32, _i32, _vp, _i32, _vp]),
     "lbm_nn_relu_backward": (_i32, [_vp, _vp, _vp, _i64, _vp]),

@@ -264,6 +264,38 @@ struct ConvArgs {
     int P, H, W, C, N, sign, accumulate, relu;
 };
 
+// Stores 4 consecutive output channels c of pixel p.
+__device__ __forceinline__ void conv_store(const ConvArgs &a, floatx4 v, int p, int c) {
+    if (p >= a.P) return;
+    const int64_t o = int64_t(p) * a.N + c;
+    if ((a.N & 3) == 0) {
+        if (c >= a.N) return;
+        if (a.accumulate) v += *reinterpret_cast<const floatx4 *>(a.y + o);
+        if (a.bias) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] += a.bias[c + r];
+        }
+        if (a.relu) {
+#pragma unroll
+            for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.0f);
+        }
+        if (a.y) *reinterpret_cast<floatx4 *>(a.y + o) = v;
+        if (a.yb)
+            *reinterpret_cast<ushort4 *>(a.yb + o) = make_ushort4(f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3]));
+        return;
+    }
+#pragma unroll
+    for (int r = 0; r < 4; ++r) {
+        if (c + r >= a.N) continue;
+        float u = v[r];
+        if (a.accumulate) u += a.y[o + r];
+        if (a.bias) u += a.bias[c + r];
+        if (a.relu) u = fmaxf(u, 0.0f);
+        if (a.y) a.y[o + r] = u;
+        if (a.yb) a.yb[o + r] = f2bf(u);
+    }
+}
+
 template <int MT, int NT, int D>
 __global__ __launch_bounds__(256) void k_conv3(ConvArgs a) {
     typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
@@ -341,46 +373,144 @@ __global__ __launch_bounds__(256) void k_conv3(ConvArgs a) {
         }
     }
 
-    const bool vec = (a.N & 3) == 0;
 #pragma unroll
-    for (int m = 0; m < MT; ++m) {
-        const int p = p0 + m * 16 + col;
-        if (p >= a.P) continue;
+    for (int m = 0; m < MT; ++m)
 #pragma unroll
-        for (int n = 0; n < NT; ++n) {
-            const int c = n0 + n * 16 + (lane >> 4) * 4;
-            const int64_t o = int64_t(p) * a.N + c;
-            floatx4 v = acc[m][n];
-            if (vec) {
-                if (c >= a.N) continue;
-                if (a.accumulate) v += *reinterpret_cast<const floatx4 *>(a.y + o);
-                if (a.bias) {
+        for (int n = 0; n < NT; ++n)
+            conv_store(a, acc[m][n], p0 + m * 16 + col, n0 + n * 16 + (lane >> 4) * 4);
+}
+
+// The same convolution for the network's own calls: the pixels a block's taps
+// read, one run of the flattened image, are staged in LDS once (rows of C
+// channels padded by 16 bytes, so the 16 rows of a fragment fall into different
+// banks), and the weights come packed in fragment order (k_pack_weights), 1 KB
+// of consecutive bytes a load.  k_conv3 is bound by its loads' addresses, 16
+// rows a load (some 80 cycles of a CU each, L1 hit or not); here only the staging
+// has rows to address.  Row 0 of the LDS holds zeros for pixels outside the image.
+// Waves 2 x 2: pixels 32 MT, channels 32 NT a block.
+template <int MT, int NT, int D>
+__global__ __launch_bounds__(256) void k_conv3p(ConvArgs a) {
+    typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
+    extern __shared__ __align__(16) unsigned char smem[];
+    const int t = threadIdx.x, lane = t & 63, col = lane & 15, kq = (lane >> 4) * 8;
+    const int w = __builtin_amdgcn_readfirstlane(t >> 6), wm = w >> 1, wn = w & 1;
+    const int pitch = a.C * 2 + 16;
+    const int pb = blockIdx.x * 32 * MT, r0 = pb - a.W - 1;  // pixel of LDS row 1
+    __amdgpu_buffer_rsrc_t xr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t *>(a.X), 0, int(unsigned(a.P) * unsigned(a.C) * 2u), 0x00020000);
+    const int S = 9 * (a.C / 32), per_tap = a.C / 32;
+    __amdgpu_buffer_rsrc_t wr = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t *>(a.Wt), 0, (a.N + 15) / 16 * S * 1024, 0x00020000);
+
+    u32x4 fw[D][NT];
+    unsigned wo[NT];
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] += a.bias[c + r];
-                }
-                if (a.relu) {
+    for (int n = 0; n < NT; ++n) wo[n] = unsigned(((blockIdx.y * 2 + wn) * NT + n) * S * 1024 + lane * 16);
+    auto load_w = [&](u32x4 *bw, int step) {
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) v[r] = fmaxf(v[r], 0.0f);
-                }
-                if (a.y) *reinterpret_cast<floatx4 *>(a.y + o) = v;
-                if (a.yb) {
-                    ushort4 h = make_ushort4(f2bf(v[0]), f2bf(v[1]), f2bf(v[2]), f2bf(v[3]));
-                    *reinterpret_cast<ushort4 *>(a.yb + o) = h;
-                }
-                continue;
-            }
+        for (int n = 0; n < NT; ++n)
+            bw[n] = __builtin_bit_cast(
+                u32x4, __builtin_amdgcn_raw_buffer_load_b128(wr, int(wo[n] + unsigned(step) * 1024u), 0, 0));
+    };
 #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                if (c + r >= a.N) continue;
-                float u = v[r];
-                if (a.accumulate) u += a.y[o + r];
-                if (a.bias) u += a.bias[c + r];
-                if (a.relu) u = fmaxf(u, 0.0f);
-                if (a.y) a.y[o + r] = u;
-                if (a.yb) a.yb[o + r] = f2bf(u);
-            }
+    for (int d = 0; d < D; ++d) load_w(fw[d], d);
+
+    {
+        const int cpr = a.C / 8, items = (32 * MT + 2 * a.W + 2) * cpr;
+        const float inv = 1.0f / float(cpr);
+        if (t * 16 < pitch) *reinterpret_cast<u32x4 *>(smem + t * 16) = u32x4{0, 0, 0, 0};
+#pragma unroll 4
+        for (int i = t; i < items; i += 256) {
+            const int r = int((float(i) + 0.5f) * inv), c = i - r * cpr;
+            const int q = r0 + r;
+            const unsigned o = q >= 0 && q < a.P ? unsigned(q) * unsigned(a.C) * 2u + unsigned(c) * 16u : 0x80000000u;
+            *reinterpret_cast<u32x4 *>(smem + (r + 1) * pitch + c * 16) =
+                __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(xr, int(o), 0, 0));
         }
     }
+
+    unsigned in[MT];
+    int base[MT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m) {
+        const int lp = (wm * MT + m) * 16 + col, p = pb + lp;
+        const int x = p % a.W, y = (p / a.W) % a.H;
+        unsigned bits = 0;
+#pragma unroll
+        for (int tap = 0; tap < 9; ++tap) {
+            const int yy = y + a.sign * (tap / 3 - 1), xx = x + a.sign * (tap % 3 - 1);
+            bits |= unsigned(p < a.P && unsigned(yy) < unsigned(a.H) && unsigned(xx) < unsigned(a.W)) << tap;
+        }
+        in[m] = bits;
+        base[m] = (lp + a.W + 2) * pitch + kq * 2;
+    }
+    floatx4 acc[MT][NT];
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n) acc[m][n] = floatx4{0.f, 0.f, 0.f, 0.f};
+    __syncthreads();
+
+    int tap = 0, cc = 0, at[MT];
+    for (int s = 0; s < S; s += D) {
+#pragma unroll
+        for (int d = 0; d < D; ++d) {
+            if (cc == 0) {
+                const int shift = a.sign * ((tap / 3 - 1) * a.W + (tap % 3 - 1)) * pitch;
+#pragma unroll
+                for (int m = 0; m < MT; ++m) at[m] = (in[m] >> tap) & 1u ? base[m] + shift : kq * 2;
+            }
+            bf16x8 x[MT];
+#pragma unroll
+            for (int m = 0; m < MT; ++m) x[m] = *reinterpret_cast<const bf16x8 *>(smem + at[m] + cc * 64);
+#pragma unroll
+            for (int m = 0; m < MT; ++m)
+#pragma unroll
+                for (int n = 0; n < NT; ++n)
+                    acc[m][n] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(__builtin_bit_cast(bf16x8, fw[d][n]), x[m],
+                                                                        acc[m][n], 0, 0, 0);
+            if (s + D + d < S) load_w(fw[d], s + D + d);
+            if (++cc == per_tap) cc = 0, ++tap;
+        }
+    }
+#pragma unroll
+    for (int m = 0; m < MT; ++m)
+#pragma unroll
+        for (int n = 0; n < NT; ++n)
+            conv_store(a, acc[m][n], pb + (wm * MT + m) * 16 + col,
+                       ((blockIdx.y * 2 + wn) * NT + n) * 16 + (lane >> 4) * 4);
+}
+
+// Weights of several layers in the fragment order of k_conv3p: for output channel
+// tile i and 32-channel step s, lane l holds channels k = 32 s + (l / 16) 8 .. + 7 of
+// output i 16 + l % 16 (zero past the last).  forward: output co, k = tap cin + c;
+// transposed (the data gradient): output c, k = tap cout + co.
+struct PackTable {
+    int n, transposed;
+    int64_t from[LBM_NN_MAX_LAYERS], to[LBM_NN_MAX_LAYERS];  // elements
+    int cin[LBM_NN_MAX_LAYERS], cout[LBM_NN_MAX_LAYERS], first[LBM_NN_MAX_LAYERS + 1];
+};
+
+__global__ __launch_bounds__(256) void k_pack_weights(const uint16_t *__restrict__ w, uint16_t *__restrict__ out,
+                                                      const PackTable q) {
+    int j = 0;
+    while (int(blockIdx.x) >= q.first[j + 1]) ++j;
+    const int cin = q.cin[j], cout = q.cout[j];
+    const int K = q.transposed ? cout : cin, N = q.transposed ? cin : cout, S = 9 * K / 32;
+    const int i = (int(blockIdx.x) - q.first[j]) * 256 + int(threadIdx.x);  // (tile, step, lane)
+    if (i >= (N + 15) / 16 * S * 64) return;
+    const int lane = i & 63, s = (i >> 6) % S, n = (i >> 6) / S * 16 + (lane & 15);
+    const int k = s * 32 + (lane >> 4) * 8, tap = k / K, c = k - tap * K;
+    const uint16_t *src = w + q.from[j];
+    uint16_t v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        v[e] = 0;
+        if (n < N) v[e] = q.transposed ? src[(int64_t(c + e) * 9 + tap) * cin + n] : src[(int64_t(n) * 9 + tap) * cin + c + e];
+    }
+    uint4 o = make_uint4(v[0] | unsigned(v[1]) << 16, v[2] | unsigned(v[3]) << 16, v[4] | unsigned(v[5]) << 16,
+                         v[6] | unsigned(v[7]) << 16);
+    *reinterpret_cast<uint4 *>(out + q.to[j] + int64_t(i) * 8) = o;
 }
 
 // Weight gradient of the 3x3 convolution: dW[co][tap * C + c] = sum over pixels
@@ -796,7 +926,7 @@ __global__ __launch_bounds__(256) void k_avgpool2(const float *__restrict__ x, i
     Vec<V> r;
 #pragma unroll
     for (int i = 0; i < V; ++i) r.v[i] = 0.25f * ((q0.v[i] + q1.v[i]) + (q2.v[i] + q3.v[i]));
-    r.store(y + idx * V);
+    if (y) r.store(y + idx * V);
     if (yb) r.store_bf16(yb + idx * V);
 }
 
@@ -850,6 +980,21 @@ __global__ __launch_bounds__(256) void k_upsample2_backward(const float *__restr
         for (int i = 0; i < V; ++i) s.v[i] += g.v[i];
     }
     s.store(dx + idx * V);
+}
+
+// The decoder's input in BF16: nearest 2x upsample of h [B][H][W][Ch], then skip
+// [B][2H][2W][Cs], V channels (16 bytes, or one) a thread.
+template <int V>
+__global__ __launch_bounds__(256) void k_concat_up(const uint16_t *__restrict__ h, const uint16_t *__restrict__ skip,
+                                                   int64_t items, int H, int W, int Ch, int Cs,
+                                                   uint16_t *__restrict__ out) {
+    const int64_t idx = int64_t(blockIdx.x) * 256 + threadIdx.x;
+    if (idx >= items) return;
+    const Pixel o(idx, (Ch + Cs) / V, V, 2 * H, 2 * W);
+    const uint16_t *src = o.c < Ch ? h + ((int64_t(o.b) * H + o.y / 2) * W + o.x / 2) * Ch + o.c
+                                   : skip + o.p * Cs + (o.c - Ch);
+    if constexpr (V == 8) *reinterpret_cast<uint4 *>(out + idx * 8) = *reinterpret_cast<const uint4 *>(src);
+    else out[idx] = *src;
 }
 
 // Channel-slice copy: dst[p][doff + c] (+)= src[p][soff + c] for c < C.
@@ -1183,7 +1328,240 @@ static int run_conv(const ConvArgs &a, hipStream_t s) {
     return launch_status();
 }
 
+// LDS of k_conv3p at 32 mt pixels a block, and the most a block may take: two
+// share a CU.
+static int64_t conv_lds(const ConvArgs &a, int mt) {
+    return (int64_t(32) * mt + 2 * int64_t(a.W) + 3) * (2 * a.C + 16);
+}
+constexpr int64_t kConvLds = 80 * 1024;
+
+static bool conv_packed_fits(const ConvArgs &a) {
+    const int64_t step_bytes = (int64_t(a.N) + 15) / 16 * (9 * a.C / 32) * 1024;
+    return conv_direct(a) && conv_lds(a, 1) <= kConvLds && step_bytes < (int64_t(1) << 31);
+}
+
+template <int MT, int NT, int D>
+static int launch_conv_packed(const ConvArgs &a, hipStream_t s) {
+    const dim3 grid(unsigned((a.P + 32 * MT - 1) / (32 * MT)), unsigned((a.N + 32 * NT - 1) / (32 * NT)));
+    hipLaunchKernelGGL((k_conv3p<MT, NT, D>), grid, dim3(256), unsigned(conv_lds(a, MT)), s, a);
+    return launch_status();
+}
+
+static int run_conv_packed(const ConvArgs &a, hipStream_t s) {
+    // us of the whole layer, batch 16 of a 128 x 128 network unless said otherwise,
+    // against the best tile of k_conv3:
+    //   128 pixels x 32 channels while that gives every CU eight blocks: few
+    //     channels, where staging weighs most (32 -> 32 at 128^2: 26.9, 2 x 2
+    //     tiles 31.0, k_conv3 26.8; 96 -> 32: 62.5, 102, 59);
+    //   64 x 64 while every CU gets a block (256 -> 128 at 32^2: 18.9 against
+    //     54, 513 TFLOP/s; 128 -> 128: 13.0 against 31; 64 -> 64 at 64^2: 16.6
+    //     against 27);
+    //   32 x 32 below, the weights of nine steps in flight (128 -> 128 at 16^2: 7.7
+    //     against 15; batch 1, 256 -> 128 at 32^2: 10.7 against 18.3).
+    const int64_t cus = device_cus();
+    auto blocks = [&](int mt, int nt) {
+        return int64_t((a.P + 32 * mt - 1) / (32 * mt)) * ((a.N + 32 * nt - 1) / (32 * nt));
+    };
+    if (a.N <= 96 && conv_lds(a, 4) <= kConvLds && blocks(4, 1) >= 8 * cus) return launch_conv_packed<4, 1, 3>(a, s);
+    if (conv_lds(a, 2) <= kConvLds && blocks(2, 2) >= cus) return launch_conv_packed<2, 2, 3>(a, s);
+    return launch_conv_packed<1, 1, 9>(a, s);
+}
+
 extern "C" {
+
+int lbm_nn_packed_fits(int B, int H, int W, int cin, int cout) {
+    const int64_t P = int64_t(B) * H * W;
+    if (B <= 0 || H <= 0 || W <= 0 || cin <= 0 || cout <= 0 || P * 9 * cin >= (int64_t(1) << 31) ||
+        P * cout >= (int64_t(1) << 31))
+        return 0;
+    const ConvArgs a{nullptr, nullptr, nullptr, nullptr, nullptr, int(P), H, W, cin, cout, 1, 0, 0};
+    return conv_packed_fits(a);
+}
+
+int64_t lbm_nn_packed_size(int cin, int cout) {
+    if (cin <= 0 || cout <= 0) return LBM_E_SIZE;
+    // either orientation; 0 where the packed kernels do not apply
+    const int64_t f = cin % 32 ? 0 : (int64_t(cout) + 15) / 16 * 16 * 9 * cin;
+    const int64_t t = cout % 32 ? 0 : (int64_t(cin) + 15) / 16 * 16 * 9 * cout;
+    return f > t ? f : t;
+}
+
+int lbm_nn_pack_weights(const void *w, const int64_t *from, const int *cin, const int *cout, int n,
+                        int transposed, void *out, const int64_t *to, void *stream) {
+    if (!w || !from || !cin || !cout || !out || !to) return LBM_E_NULL;
+    if (n <= 0 || n > LBM_NN_MAX_LAYERS) return LBM_E_SIZE;
+    if (reinterpret_cast<uintptr_t>(out) % 16) return LBM_E_ARG;
+    PackTable q{};
+    q.transposed = transposed;
+    for (int i = 0; i < n; ++i) {
+        if (cin[i] <= 0 || cout[i] <= 0 || int64_t(cin[i]) * cout[i] > (int64_t(1) << 26)) return LBM_E_SIZE;
+        if (from[i] < 0 || to[i] < 0 || to[i] % 8) return LBM_E_ARG;
+        const int K = transposed ? cout[i] : cin[i], N = transposed ? cin[i] : cout[i];
+        if (K % 32) continue;
+        const int j = q.n++;
+        q.from[j] = from[i], q.to[j] = to[i], q.cin[j] = cin[i], q.cout[j] = cout[i];
+        q.first[j + 1] = q.first[j] + ((N + 15) / 16 * (9 * K / 32) * 64 + 255) / 256;
+    }
+    if (q.n == 0) return LBM_OK;
+    hipLaunchKernelGGL(k_pack_weights, dim3(unsigned(q.first[q.n])), dim3(256), 0, as_stream(stream),
+                       static_cast<const uint16_t *>(w), static_cast<uint16_t *>(out), q);
+    return launch_status();
+}
+
+}  // extern "C"
+
+// The U-Net's layers and the buffers of one forward pass.
+namespace {
+struct Unet {
+    struct Layer {
+        int cin, cout, level;
+        int64_t w, wp;  // element offsets in the flat parameters, in the packed ones
+    };
+    Layer layer[LBM_NN_MAX_LAYERS];
+    int n = 0, levels = 0;
+    int64_t packed = 0, bytes = 0;
+    int64_t xb, encf, enca[8], skip[8], pool[8], mida, midb, cat[8], deca[8], decb[8];  // byte offsets
+};
+
+int64_t take(Unet &u, int64_t bytes) {
+    const int64_t at = u.bytes;
+    u.bytes += (bytes + 255) / 256 * 256;
+    return at;
+}
+
+bool plan_unet(Unet &u, int B, int H, int W, int in_ch, const int *widths, int levels, int mid, int out_ch) {
+    if (B <= 0 || H <= 0 || W <= 0 || in_ch <= 0 || mid <= 0 || out_ch <= 0 || !widths || levels < 1 ||
+        levels > 7 || 4 * levels + 3 > LBM_NN_MAX_LAYERS || H % (1 << levels) || W % (1 << levels))
+        return false;
+    for (int i = 0; i < levels; ++i)
+        if (widths[i] <= 0) return false;
+    u.levels = levels;
+    int64_t flat = 0;
+    auto add = [&](int cin, int cout, int level) {
+        u.layer[u.n++] = Unet::Layer{cin, cout, level, flat, u.packed};
+        flat += int64_t(9) * cin * cout + cout;
+        if (cin % 32 == 0) u.packed += (int64_t(cout) + 15) / 16 * 16 * 9 * cin;
+    };
+    int c = in_ch;
+    for (int i = 0; i < levels; ++i) add(c, widths[i], i), add(widths[i], widths[i], i), c = widths[i];
+    add(c, mid, levels), add(mid, mid, levels), c = mid;
+    for (int i = levels - 1; i >= 0; --i) add(c + widths[i], widths[i], i), add(widths[i], widths[i], i), c = widths[i];
+    add(c, out_ch, 0);
+    const int64_t P = int64_t(B) * H * W;
+    (void)take(u, u.packed * 2);  // at 0
+    u.xb = take(u, P * in_ch * 2);
+    int64_t encf = 0;
+    for (int i = 0; i < levels; ++i) {
+        const int64_t p = P >> (2 * i);
+        encf = encf > p * widths[i] * 4 ? encf : p * widths[i] * 4;
+        u.enca[i] = take(u, p * widths[i] * 2);
+        u.skip[i] = take(u, p * widths[i] * 2);
+        u.pool[i] = take(u, p / 4 * widths[i] * 2);
+        u.cat[i] = take(u, p * ((i + 1 < levels ? widths[i + 1] : mid) + widths[i]) * 2);
+        u.deca[i] = take(u, p * widths[i] * 2);
+        u.decb[i] = take(u, p * widths[i] * 2);
+    }
+    u.encf = take(u, encf);
+    u.mida = take(u, (P >> (2 * levels)) * mid * 2);
+    u.midb = take(u, (P >> (2 * levels)) * mid * 2);
+    return true;
+}
+}  // namespace
+
+extern "C" {
+
+int64_t lbm_nn_unet_workspace(int B, int H, int W, int in_ch, const int *widths, int levels, int mid, int out_ch) {
+    Unet u;
+    return plan_unet(u, B, H, W, in_ch, widths, levels, mid, out_ch) ? u.bytes : int64_t(LBM_E_SIZE);
+}
+
+int lbm_nn_unet_forward(const float *x, int B, int H, int W, int in_ch, const int *widths, int levels, int mid,
+                        int out_ch, const float *p, const void *pb, void *work, float *out, void *stream) {
+    if (!x || !p || !pb || !work || !out) return LBM_E_NULL;
+    Unet u;
+    if (!plan_unet(u, B, H, W, in_ch, widths, levels, mid, out_ch)) return LBM_E_SIZE;
+    if (reinterpret_cast<uintptr_t>(work) % 16) return LBM_E_ARG;
+    char *const base = static_cast<char *>(work);
+    const uint16_t *const wb = static_cast<const uint16_t *>(pb);
+    int64_t from[LBM_NN_MAX_LAYERS], to[LBM_NN_MAX_LAYERS];
+    int cin[LBM_NN_MAX_LAYERS], cout[LBM_NN_MAX_LAYERS];
+    for (int i = 0; i < u.n; ++i)
+        from[i] = u.layer[i].w, to[i] = u.layer[i].wp, cin[i] = u.layer[i].cin, cout[i] = u.layer[i].cout;
+    int rc = lbm_nn_pack_weights(pb, from, cin, cout, u.n, 0, base, to, stream);
+    if (!rc) rc = lbm_nn_to_bf16(x, base + u.xb, int64_t(B) * H * W * in_ch, stream);
+    int next = 0;
+    auto conv = [&](int64_t src, float *y, void *yb, bool relu) {
+        const Unet::Layer &l = u.layer[next++];
+        if (rc) return;
+        const uint16_t *wp = l.cin % 32 ? nullptr : reinterpret_cast<const uint16_t *>(base) + l.wp;
+        rc = lbm_nn_conv3x3_packed(base + src, B, H >> l.level, W >> l.level, l.cin, wb + l.w, wp, l.cout,
+                                   p + l.w + int64_t(9) * l.cin * l.cout, y, yb, relu, stream);
+    };
+    float *const f32 = reinterpret_cast<float *>(base + u.encf);
+    int64_t h = u.xb;
+    for (int i = 0; i < levels; ++i) {
+        conv(h, nullptr, base + u.enca[i], true);
+        conv(u.enca[i], f32, base + u.skip[i], true);  // the pool averages the FP32 values
+        const int hh = H >> i, ww = W >> i, c = widths[i];
+        if (rc) return rc;
+        const int64_t n = int64_t(B) * (hh / 2) * (ww / 2) * c;
+        uint16_t *const pooled = reinterpret_cast<uint16_t *>(base + u.pool[i]);
+        if (by_four({c}, {f32}, pooled))
+            hipLaunchKernelGGL(k_avgpool2<4>, dim3(blocks_for(n / 4)), dim3(256), 0, as_stream(stream), f32, B, hh,
+                               ww, c, static_cast<float *>(nullptr), pooled);
+        else
+            hipLaunchKernelGGL(k_avgpool2<1>, dim3(blocks_for(n)), dim3(256), 0, as_stream(stream), f32, B, hh, ww,
+                               c, static_cast<float *>(nullptr), pooled);
+        h = u.pool[i];
+    }
+    conv(h, nullptr, base + u.mida, true);
+    conv(u.mida, nullptr, base + u.midb, true);
+    h = u.midb;
+    for (int i = levels - 1; i >= 0; --i) {
+        if (rc) return rc;
+        const int ch = i + 1 < levels ? widths[i + 1] : mid, cs = widths[i];
+        const int64_t n = int64_t(B) * (H >> i) * (W >> i) * (ch + cs);
+        const uint16_t *hp = reinterpret_cast<const uint16_t *>(base + h);
+        const uint16_t *sp = reinterpret_cast<const uint16_t *>(base + u.skip[i]);
+        uint16_t *cp = reinterpret_cast<uint16_t *>(base + u.cat[i]);
+        if (ch % 8 == 0 && cs % 8 == 0)
+            hipLaunchKernelGGL(k_concat_up<8>, dim3(blocks_for(n / 8)), dim3(256), 0, as_stream(stream), hp, sp,
+                               n / 8, H >> (i + 1), W >> (i + 1), ch, cs, cp);
+        else
+            hipLaunchKernelGGL(k_concat_up<1>, dim3(blocks_for(n)), dim3(256), 0, as_stream(stream), hp, sp, n,
+                               H >> (i + 1), W >> (i + 1), ch, cs, cp);
+        conv(u.cat[i], nullptr, base + u.deca[i], true);
+        conv(u.deca[i], nullptr, base + u.decb[i], true);
+        h = u.decb[i];
+    }
+    conv(h, out, nullptr, false);
+    return rc ? rc : launch_status();
+}
+
+int lbm_nn_conv3x3_packed(const void *x, int B, int H, int W, int cin, const void *w, const void *wp, int cout,
+                          const float *bias, float *y, void *yb, int relu, void *stream) {
+    if (!x || !w || (!y && !yb)) return LBM_E_NULL;
+    if (B <= 0 || H <= 0 || W <= 0 || cin <= 0 || cout <= 0) return LBM_E_SIZE;
+    const int64_t P = int64_t(B) * H * W;
+    if (wp && P * 9 * cin < (int64_t(1) << 31) && P * cout < (int64_t(1) << 31)) {
+        const ConvArgs a{static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(wp), y,
+                         static_cast<uint16_t *>(yb), bias, int(P), H, W, cin, cout, 1, 0, relu};
+        if (conv_packed_fits(a)) return run_conv_packed(a, as_stream(stream));
+    }
+    return lbm_nn_conv3x3(x, B, H, W, cin, w, cout, bias, y, yb, relu, stream);
+}
+
+int lbm_nn_conv3x3_dgrad_packed(const void *dy, const void *wp, int B, int H, int W, int cin, int cout,
+                                float *dx, void *stream) {
+    if (!dy || !wp || !dx) return LBM_E_NULL;
+    if (B <= 0 || H <= 0 || W <= 0 || cin <= 0 || cout <= 0) return LBM_E_SIZE;
+    const int64_t P = int64_t(B) * H * W;
+    if (P * 9 * cout >= (int64_t(1) << 31) || P * cin >= (int64_t(1) << 31)) return LBM_E_SIZE;
+    const ConvArgs a{static_cast<const uint16_t *>(dy), static_cast<const uint16_t *>(wp), dx, nullptr,
+                     nullptr, int(P), H, W, cout, cin, -1, 0, 0};
+    if (!conv_packed_fits(a)) return LBM_E_ARG;
+    return run_conv_packed(a, as_stream(stream));
+}
 
 int64_t lbm_nn_gemm_workspace(int M, int N, int ksplit) {
     return ksplit > 1 ? int64_t(ksplit) * M * N * int64_t(sizeof(float)) : 0;

@@ -17,6 +17,7 @@ concatenation with the level's skip, and two ReLU convolutions on the way up,
 then a linear 3x3 head.
 """
 
+import ctypes
 import math
 
 import numpy as np
@@ -59,6 +60,18 @@ class Surrogate:
             self.offsets[name] = (n, n + 9 * cin * cout)
             n += 9 * cin * cout + cout
         self.nparams = n
+        # tables of the native calls: widths; weight offsets, channels and packed
+        # places of every layer
+        k = len(self.layers)
+        self._widths = (ctypes.c_int * len(self.widths))(*self.widths)
+        self._from = (ctypes.c_int64 * k)(*(self.offsets[l[0]][0] for l in self.layers))
+        self._cin = (ctypes.c_int * k)(*(l[1] for l in self.layers))
+        self._cout = (ctypes.c_int * k)(*(l[2] for l in self.layers))
+        self._to, self.packed, size = (ctypes.c_int64 * k)(), {}, 0
+        for i, (name, cin, cout, _) in enumerate(self.layers):
+            self._to[i] = self.packed[name] = size
+            size += int(nat.load().lbm_nn_packed_size(cin, cout))
+        self._packed_size = size
         f32 = dict(dtype=torch.float32, device=self.device)
         self.p = torch.empty(n, **f32)
         self.pb = torch.empty(n, dtype=torch.bfloat16, device=self.device)
@@ -110,8 +123,25 @@ class Surrogate:
         net.load_flat(state["flat"])
         return net
 
+    def _pack(self, transposed):
+        """The BF16 weights in the fragment order of the convolution kernels, for
+        the forward pass or the data gradients."""
+        wp = torch.empty(max(8, self._packed_size), dtype=torch.bfloat16, device=self.device)
+        if len(self.layers) <= nat.NN_MAX_LAYERS:
+            nat.call("lbm_nn_pack_weights", _p(self.pb), ctypes.addressof(self._from),
+                     ctypes.addressof(self._cin), ctypes.addressof(self._cout), len(self.layers),
+                     int(transposed), _p(wp), ctypes.addressof(self._to), nat.stream_ptr())
+        return wp
+
+    def _packed_ptr(self, wp, name, k):
+        """Address of the layer's packed weights, None where they do not apply
+        (``k`` channels summed over)."""
+        if wp is None or k % 32 or len(self.layers) > nat.NN_MAX_LAYERS:
+            return None
+        return _p(wp) + 2 * self.packed[name]
+
     # -- building blocks ----------------------------------------------------------
-    def _conv(self, name, x, xb, relu=None):
+    def _conv(self, name, x, xb, relu=None, packed=None):
         B, H, W, cin = x.shape
         cin_, cout, relu_ = self.spec[name]
         assert cin == cin_, (name, cin, cin_)
@@ -119,8 +149,9 @@ class Surrogate:
         y = torch.empty((B, H, W, cout), dtype=torch.float32, device=self.device)
         yb = torch.empty((B, H, W, cout), dtype=torch.bfloat16, device=self.device)
         wb, bias = self.views(name, self.pb)[0], self.views(name)[1]
-        nat.call("lbm_nn_conv3x3", _p(xb), B, H, W, cin, _p(wb), cout, _p(bias), _p(y), _p(yb),
-                 int(relu), nat.stream_ptr())
+        nat.call("lbm_nn_conv3x3_packed", _p(xb), B, H, W, cin, _p(wb),
+                 self._packed_ptr(packed, name, cin), cout, _p(bias), _p(y), _p(yb), int(relu),
+                 nat.stream_ptr())
         return y, yb
 
     def _pool(self, x):
@@ -151,12 +182,22 @@ class Surrogate:
         if C != self.in_ch or H % (1 << lv) or W % (1 << lv):
             raise ValueError("input must be (B, H, W, %d) with H, W divisible by %d"
                              % (self.in_ch, 1 << lv))
+        if not keep and 1 <= lv <= 7 and x.numel():
+            # BF16 activations only (what the GEMMs read), launched natively
+            dims = (B, H, W, C, ctypes.addressof(self._widths), lv, self.mid, self.out_ch)
+            work = torch.empty(int(nat.load().lbm_nn_unet_workspace(*dims)), dtype=torch.uint8,
+                               device=self.device)
+            out = torch.empty((B, H, W, self.out_ch), dtype=torch.float32, device=self.device)
+            nat.call("lbm_nn_unet_forward", _p(x), *dims, _p(self.p), _p(self.pb), _p(work), _p(out),
+                     nat.stream_ptr())
+            return out
         xb = torch.empty_like(x, dtype=torch.bfloat16)
         nat.call("lbm_nn_to_bf16", _p(x), _p(xb), x.numel(), nat.stream_ptr())
         cache = {}
+        packed = self._pack(False)
 
         def conv(name, h, hb):
-            y, yb = self._conv(name, h, hb)
+            y, yb = self._conv(name, h, hb, packed=packed)
             if keep:
                 cache[name] = (hb, y, tuple(h.shape))
             return y, yb
@@ -176,7 +217,7 @@ class Surrogate:
         out, _ = conv("head", h, hb)
         return (out, cache) if keep else out
 
-    def _back(self, cache, name, dy, need_dx=True):
+    def _back(self, cache, name, dy, need_dx=True, packed=None):
         xb, y, (B, H, W, cin) = cache[name]
         _, cout, relu = self.spec[name]
         P, K = B * H * W, 9 * cin
@@ -199,6 +240,11 @@ class Surrogate:
         if not need_dx:
             return None
         # dx[p][c] = sum over taps and co of dy[p - tap][co] W[co][tap][c]
+        wp = self._packed_ptr(packed, name, cout)
+        if wp is not None and nat.load().lbm_nn_packed_fits(B, H, W, cout, cin):
+            dx = torch.empty((B, H, W, cin), dtype=torch.float32, device=self.device)
+            nat.call("lbm_nn_conv3x3_dgrad_packed", _p(dyb), wp, B, H, W, cin, cout, _p(dx), s)
+            return dx
         wb = self.views(name, self.pb)[0]
         wf = torch.empty(9 * cin * cout, dtype=torch.bfloat16, device=self.device)
         nat.call("lbm_nn_conv3x3_transpose_weights", _p(wb), cin, cout, _p(wf), s)
@@ -210,11 +256,16 @@ class Surrogate:
         """Fill the gradient buffer from dL/d(output); optionally return dL/d(input)."""
         s = nat.stream_ptr()
         lv = len(self.widths)
-        g = self._back(cache, "head", dout)
+        packed = self._pack(True)
+
+        def back(name, dy, need_dx=True):
+            return self._back(cache, name, dy, need_dx, packed)
+
+        g = back("head", dout)
         dskips = [None] * lv
         for i in range(lv):
-            g = self._back(cache, "dec%db" % i, g)
-            g = self._back(cache, "dec%da" % i, g)
+            g = back("dec%db" % i, g)
+            g = back("dec%da" % i, g)
             B, H, W, Ct = g.shape
             Cs = self.widths[i]
             Ch = Ct - Cs
@@ -222,8 +273,8 @@ class Surrogate:
             gu = torch.empty((B, H // 2, W // 2, Ch), dtype=torch.float32, device=self.device)
             nat.call("lbm_nn_upsample2_backward", _p(g), B, H // 2, W // 2, Ch, Ct, 0, _p(gu), s)
             g = gu
-        g = self._back(cache, "midb", g)
-        g = self._back(cache, "mida", g)
+        g = back("midb", g)
+        g = back("mida", g)
         for i in reversed(range(lv)):
             B, h2, w2, C = g.shape
             gs = torch.empty((B, 2 * h2, 2 * w2, C), dtype=torch.float32, device=self.device)
@@ -232,8 +283,8 @@ class Surrogate:
             Ct = cat.shape[3]
             nat.call("lbm_nn_copy_channels", _p(cat), Ct, Ct - C, _p(gs), None, C, 0, C,
                      B * 4 * h2 * w2, 1, s)
-            g = self._back(cache, "enc%db" % i, gs)
-            g = self._back(cache, "enc%da" % i, g, need_dx=need_input_grad or i > 0)
+            g = back("enc%db" % i, gs)
+            g = back("enc%da" % i, g, need_dx=need_input_grad or i > 0)
         return g
 
     def mse(self, out, target):

@@ -521,3 +521,67 @@ def test_conv3x3_direct_kernels(gpu, B, H, W, cin, cout):
     assert lib.lbm_nn_conv3x3_wgrad_splits(0, 1, 1, 1, 1) == -2
     assert lib.lbm_nn_conv3x3_transpose_weights(None, cin, cout, _p(wt), sp) == -1
     assert lib.lbm_nn_conv3x3_dgrad_t(None, _p(wt), B, H, W, cin, cout, _p(dx), 0, sp) == -1
+
+
+# pixels and channels around the block tiles, images whose rows leave the LDS no
+# room (W = 700: unpacked form), each of the three block shapes in both directions
+@pytest.mark.parametrize("B,H,W,cin,cout", [(1, 16, 17, 32, 3), (3, 9, 11, 64, 96), (2, 13, 10, 96, 40),
+                                            (1, 8, 8, 256, 128), (6, 64, 64, 64, 64), (17, 128, 128, 32, 32),
+                                            (1, 3, 700, 96, 32)])
+def test_conv3x3_packed_kernels(gpu, B, H, W, cin, cout):
+    import ctypes
+    nat = _nat()
+    rng = np.random.default_rng(cin + cout + W)
+    P, sp, lib = B * H * W, nat.stream_ptr(), nat.load()
+    x, _ = _bf(rng, (B, H, W, cin))
+    w, _ = _bf(rng, (2, cout, 3, 3, cin), 0.2)  # two layers, packed in one launch
+    dy, _ = _bf(rng, (B, H, W, cout))
+    bias = torch.as_tensor(rng.normal(size=cout).astype(np.float32)).cuda()
+    n = int(lib.lbm_nn_packed_size(cin, cout))
+    frm, to = (ctypes.c_int64 * 2)(0, w[0].numel()), (ctypes.c_int64 * 2)(0, n)
+    ci, co = (ctypes.c_int * 2)(cin, cin), (ctypes.c_int * 2)(cout, cout)
+    for transposed in (0, 1):
+        if (cout if transposed else cin) % 32:
+            continue
+        wp = torch.full((2 * n,), float("nan"), dtype=torch.bfloat16, device="cuda")
+        nat.call("lbm_nn_pack_weights", _p(w), ctypes.addressof(frm), ctypes.addressof(ci),
+                 ctypes.addressof(co), 2, transposed, _p(wp), ctypes.addressof(to), sp)
+        wp1 = wp[n:]
+        if not transposed:
+            y, ye = (torch.full((P, cout), -1.0, device="cuda") for _ in range(2))
+            yb, yeb = (torch.empty((P, cout), dtype=torch.bfloat16, device="cuda") for _ in range(2))
+            nat.call("lbm_nn_conv3x3", _p(x), B, H, W, cin, _p(w[1]), cout, _p(bias), _p(ye), _p(yeb), 1, sp)
+            nat.call("lbm_nn_conv3x3_packed", _p(x), B, H, W, cin, _p(w[1]), _p(wp1), cout, _p(bias), _p(y),
+                     _p(yb), 1, sp)
+            assert torch.equal(y, ye) and torch.equal(yb, yeb)
+            nat.call("lbm_nn_conv3x3_packed", _p(x), B, H, W, cin, _p(w[1]), _p(wp1), cout, None, None,
+                     _p(yb), 0, sp)
+            nat.call("lbm_nn_conv3x3", _p(x), B, H, W, cin, _p(w[1]), cout, None, None, _p(yeb), 0, sp)
+            assert torch.equal(yb, yeb)
+        else:
+            wt = torch.empty(9 * cin * cout, dtype=torch.bfloat16, device="cuda")
+            nat.call("lbm_nn_conv3x3_transpose_weights", _p(w[1]), cin, cout, _p(wt), sp)
+            dx, dxe = (torch.empty((P, cin), device="cuda") for _ in range(2))
+            nat.call("lbm_nn_conv3x3_dgrad_t", _p(dy), _p(wt), B, H, W, cin, cout, _p(dxe), 0, sp)
+            status = lib.lbm_nn_conv3x3_dgrad_packed(_p(dy), _p(wp1), B, H, W, cin, cout, _p(dx), sp)
+            if lib.lbm_nn_packed_fits(B, H, W, cout, cin):
+                assert status == 0 and torch.equal(dx, dxe)
+            else:
+                assert status == -3
+    assert lib.lbm_nn_packed_fits(1, 3, 700, 96, 32) == 0 and lib.lbm_nn_packed_size(0, 1) == -2
+
+
+@pytest.mark.parametrize("in_ch,widths,mid,B,H,W", [(18, (32, 64, 128), 128, 2, 72, 64), (5, (8, 40), 24, 1, 12, 20),
+                                                    (6, (7,), 9, 3, 6, 10), (4, (), 16, 1, 5, 7)])
+def test_native_forward_equals_kept_forward(gpu, in_ch, widths, mid, B, H, W):
+    from latticeboltzmann_amd.warmstart.network import Surrogate
+    net = Surrogate(in_ch=in_ch, widths=widths, mid=mid, seed=3)
+    x = torch.randn(B, H, W, in_ch, device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    kept, cache = net.forward(x, keep=True)
+    assert torch.equal(net.forward(x), kept)
+    net.p.mul_(0.5)
+    net.sync_bf16()
+    again, _ = net.forward(x, keep=True)
+    assert torch.equal(net.forward(x), again) and not torch.equal(again, kept)
+    lib = _nat().load()
+    assert lib.lbm_nn_unet_workspace(1, 5, 8, 4, None, 1, 8, 3) == -2
