@@ -95,15 +95,18 @@ __global__ __launch_bounds__(BS) void k_batch_step(const typename Codec<FMT>::ra
 // rounded with the batch's dither (the step's seed combined on the device
 // with *epoch; node = instance offset / 9 + k ny + l), so a launch is bitwise
 // K lbm_batch_step launches.  Instances need ny >= 64 and nx >= 2K.
-template <int FMT, typename CT, int K>
+// Unit: the scale is 1 (FP32 storage), and the 18 products with it and its inverse
+// that a node's step would take fall away.
+template <int FMT, typename CT, int K, bool Unit>
 __global__ __launch_bounds__(256) void k_batch_sweep(const typename Codec<FMT>::raw *__restrict__ src,
                                                      typename Codec<FMT>::raw *__restrict__ dst,
                                                      const lbm_batch_inst *__restrict__ insts,
                                                      const lbm_batch_item *__restrict__ items,
-                                                     int nitems, int nblocks, CT scale, CT inv_scale,
+                                                     int nitems, int nblocks, CT scale_in, CT inv_scale_in,
                                                      int stochastic, uint32_t seed,
                                                      uint32_t seed_stride,
                                                      const uint32_t *__restrict__ epoch) {
+    const CT scale = Unit ? CT(1) : scale_in, inv_scale = Unit ? CT(1) : inv_scale_in;
     const int b = xcd_tile(nblocks);
     const int w = __builtin_amdgcn_readfirstlane(b * 4 + int(threadIdx.x >> 6));
     if (b >= nblocks || w >= nitems) return;  // whole waves; nothing waits for them
@@ -257,9 +260,15 @@ void launch_batch_sweep_v(const void *src, void *dst, float scale, const lbm_bat
     using R = typename Codec<FMT>::raw;
     const int nblocks = (nitems + 3) / 4;
     const int grid = ((nblocks + 7) / 8) * 8;
-    hipLaunchKernelGGL((k_batch_sweep<FMT, CT, K>), dim3(unsigned(grid)), dim3(256), 0, s,
-                       static_cast<const R *>(src), static_cast<R *>(dst), insts, items, nitems,
-                       nblocks, CT(scale), CT(1) / CT(scale), stochastic, seed, stride, epoch);
+    auto launch = [&](auto kernel) {
+        hipLaunchKernelGGL(kernel, dim3(unsigned(grid)), dim3(256), 0, s, static_cast<const R *>(src),
+                           static_cast<R *>(dst), insts, items, nitems, nblocks, CT(scale),
+                           CT(1) / CT(scale), stochastic, seed, stride, epoch);
+    };
+    if constexpr (FMT == LBM_FMT_F32) {
+        if (scale == 1.0f) return launch(k_batch_sweep<FMT, CT, K, true>);
+    }
+    launch(k_batch_sweep<FMT, CT, K, false>);
 }
 
 template <typename CT, int K>

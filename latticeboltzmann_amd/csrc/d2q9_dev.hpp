@@ -402,6 +402,23 @@ __device__ __forceinline__ void dev_sweep_walls(CT g[9], const CT c[9], int k, i
     }
 }
 
+// What the sweep keeps of an intermediate step.  Rounded every step with an FP64
+// collide, the values are storage values: kept as FP32 (which holds every format's
+// exactly) they take half the registers and half the lane exchanges of the FP64
+// values they decode to, and decode to the same bits when they are pulled.
+template <int FMT, typename CT, bool EACH>
+struct SweepValue {
+    using type = CT;
+    __device__ static CT keep(typename Codec<FMT>::raw q, CT inv_scale) { return CT(Codec<FMT>::dec(q)) * inv_scale; }
+    __device__ static CT pull(CT v, CT) { return v; }
+};
+template <int FMT>
+struct SweepValue<FMT, double, true> {
+    using type = float;
+    __device__ static float keep(typename Codec<FMT>::raw q, double) { return Codec<FMT>::dec(q); }
+    __device__ static double pull(float v, double inv_scale) { return double(v) * inv_scale; }
+};
+
 struct DevSweepLane {
     int l, from_lo, from_hi;
     bool writer, yedge;
@@ -412,15 +429,20 @@ __device__ __forceinline__ void dev_sweep_iteration(
     const typename Codec<FMT>::raw *__restrict__ src, typename Codec<FMT>::raw *__restrict__ dst,
     int i, int ks, int nx, int ny, Layout L, const DevSweepLane &ln, CT omega, CT u0, CT scale,
     CT inv_scale, int stochastic, const uint32_t (&seeds)[K], uint64_t node_base,
-    CT (&A)[K - 1][9], CT (&B)[K - 1][9], float *__restrict__ ux_o, float *__restrict__ uy_o) {
+    typename SweepValue<FMT, CT, EACH>::type (&A)[K - 1][9],
+    typename SweepValue<FMT, CT, EACH>::type (&B)[K - 1][9], float *__restrict__ ux_o,
+    float *__restrict__ uy_o) {
     using C = Codec<FMT>;
     using R = typename C::raw;
-    CT g[9];
+    using V = SweepValue<FMT, CT, EACH>;
+    using ST = typename V::type;
+    ST made[9];  // the row the last step made
     {  // step 1 of row i + K - 1, from src
         const int k = wrap1(i + K - 1, nx);
         const PullRows<R> rows(src, L, k, nx);
         R raw[9];
         pull9<false>(rows, ln.l, ny, raw);
+        CT g[9];
 #pragma unroll
         for (int q = 0; q < 9; ++q) g[q] = CT(C::dec(raw[q])) * inv_scale;
         if constexpr (BC == LBM_BC_CAVITY) {
@@ -435,31 +457,41 @@ __device__ __forceinline__ void dev_sweep_iteration(
             R q[9];
             store_values<FMT, CT>(g, scale, stochastic, dither, q);
 #pragma unroll
-            for (int c = 0; c < 9; ++c) g[c] = CT(C::dec(q[c])) * inv_scale;
+            for (int c = 0; c < 9; ++c) made[c] = V::keep(q[c], inv_scale);
+        } else {
+#pragma unroll
+            for (int c = 0; c < 9; ++c) made[c] = g[c];
         }
     }
 #pragma unroll
     for (int j = 2; j <= K; ++j) {
-        CT(&older)[9] = PH ? B[j - 2] : A[j - 2];
-        CT(&newer)[9] = PH ? A[j - 2] : B[j - 2];
+        ST(&older)[9] = PH ? B[j - 2] : A[j - 2];
+        ST(&newer)[9] = PH ? A[j - 2] : B[j - 2];
         const bool active = i >= ks - 2 * (K - j);  // wave-uniform
         CT h[9];
         int k = 0;
         if (active) {
             k = wrap1(i + K - j, nx);
-            h[0] = newer[0];
-            h[1] = older[1];
-            h[2] = dev_lane_fetch(newer[2], ln.from_lo);
-            h[3] = g[3];
-            h[4] = dev_lane_fetch(newer[4], ln.from_hi);
-            h[5] = dev_lane_fetch(older[5], ln.from_lo);
-            h[6] = dev_lane_fetch(g[6], ln.from_lo);
-            h[7] = dev_lane_fetch(g[7], ln.from_hi);
-            h[8] = dev_lane_fetch(older[8], ln.from_hi);
-            if constexpr (BC == LBM_BC_CAVITY) dev_sweep_walls<CT>(h, newer, k, ln.l, nx, ny, u0, ln.yedge);
+            const ST p[9] = {newer[0],
+                             older[1],
+                             dev_lane_fetch(newer[2], ln.from_lo),
+                             made[3],
+                             dev_lane_fetch(newer[4], ln.from_hi),
+                             dev_lane_fetch(older[5], ln.from_lo),
+                             dev_lane_fetch(made[6], ln.from_lo),
+                             dev_lane_fetch(made[7], ln.from_hi),
+                             dev_lane_fetch(older[8], ln.from_hi)};
+#pragma unroll
+            for (int q = 0; q < 9; ++q) h[q] = V::pull(p[q], inv_scale);
+            if constexpr (BC == LBM_BC_CAVITY) {
+                CT own[9];
+#pragma unroll
+                for (int q = 0; q < 9; ++q) own[q] = V::pull(newer[q], inv_scale);
+                dev_sweep_walls<CT>(h, own, k, ln.l, nx, ny, u0, ln.yedge);
+            }
         }
 #pragma unroll
-        for (int q = 0; q < 9; ++q) older[q] = g[q];
+        for (int q = 0; q < 9; ++q) older[q] = made[q];
         if (!active) return;
         CT ux, uy;
         collide_dev<CT>(h, omega, ux, uy);
@@ -483,10 +515,10 @@ __device__ __forceinline__ void dev_sweep_iteration(
             R q[9];
             store_values<FMT, CT>(h, scale, stochastic, dither, q);
 #pragma unroll
-            for (int c = 0; c < 9; ++c) g[c] = CT(C::dec(q[c])) * inv_scale;
+            for (int c = 0; c < 9; ++c) made[c] = V::keep(q[c], inv_scale);
         } else {
 #pragma unroll
-            for (int c = 0; c < 9; ++c) g[c] = h[c];
+            for (int c = 0; c < 9; ++c) made[c] = h[c];
         }
     }
 }
@@ -500,11 +532,12 @@ __device__ __forceinline__ void dev_sweep_run(const typename Codec<FMT>::raw *__
                                               CT inv_scale, int stochastic,
                                               const uint32_t (&seeds)[K], uint64_t node_base,
                                               float *__restrict__ ux_o, float *__restrict__ uy_o) {
-    CT A[K - 1][9], B[K - 1][9];
+    using ST = typename SweepValue<FMT, CT, EACH>::type;
+    ST A[K - 1][9], B[K - 1][9];
 #pragma unroll
     for (int j = 0; j < K - 1; ++j)
 #pragma unroll
-        for (int q = 0; q < 9; ++q) A[j][q] = B[j][q] = CT(0);
+        for (int q = 0; q < 9; ++q) A[j][q] = B[j][q] = ST(0);
     int i = ks - 2 * (K - 1);
     for (; i + 1 < ke; i += 2) {
         dev_sweep_iteration<FMT, CT, BC, MOM, K, EACH, 0>(src, dst, i, ks, nx, ny, L, ln, omega, u0,
