@@ -115,6 +115,15 @@ int lbm_step_multi_f64(const double *src, double *dst, int64_t nx, int64_t ny, i
 int lbm_step_multi_f32(const float *src, float *dst, int64_t nx, int64_t ny, int layout,
                        float omega, int bc, float u0, float *rho, float *ux, float *uy,
                        int variant, void *stream);
+/* `runs` lbm_step_multi launches (multi_variant), then `single` lbm_step_layout
+ * launches (variant), from buffer a, using a and b in turn.  *in_b: which buffer
+ * holds the state after the launches made; rho/ux/uy: moments of the last step. */
+int lbm_step_run_f64(double *a, double *b, int64_t nx, int64_t ny, int layout, double omega, int bc,
+                     double u0, int64_t runs, int multi_variant, int64_t single, int variant,
+                     double *rho, double *ux, double *uy, int *in_b, void *stream);
+int lbm_step_run_f32(float *a, float *b, int64_t nx, int64_t ny, int layout, float omega, int bc,
+                     float u0, int64_t runs, int multi_variant, int64_t single, int variant,
+                     float *rho, float *ux, float *uy, int *in_b, void *stream);
 int lbm_step_multi_variant_count(void);
 int lbm_step_multi_default_variant(void); /* the FP64 tile default (below 4096^2 nodes) */
 /* The variant that -1 selects on an nx x ny grid: small tiles for grids of

@@ -71,6 +71,10 @@ SIGNATURES = {
                                   _i32, _vp]),
     "lbm_step_multi_f32": (_i32, [_vp, _vp, _i64, _i64, _i32, _f32, _i32, _f32, _vp, _vp, _vp,
                                   _i32, _vp]),
+    "lbm_step_run_f64": (_i32, [_vp, _vp, _i64, _i64, _i32, _f64, _i32, _f64, _i64, _i32, _i64, _i32,
+                                _vp, _vp, _vp, ctypes.POINTER(_i32), _vp]),
+    "lbm_step_run_f32": (_i32, [_vp, _vp, _i64, _i64, _i32, _f32, _i32, _f32, _i64, _i32, _i64, _i32,
+                                _vp, _vp, _vp, ctypes.POINTER(_i32), _vp]),
     "lbm_step_multi_variant_count": (_i32, []),
     "lbm_step_multi_default_variant": (_i32, []),
     "lbm_step_multi_default_for": (_i32, [_i64, _i64]),

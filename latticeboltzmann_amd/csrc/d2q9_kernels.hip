@@ -1101,6 +1101,28 @@ int multi_impl(const T *src, T *dst, int64_t nx, int64_t ny, int layout, T omega
     return rc ? rc : launch_status();
 }
 
+// `runs` multi-step and then `single` single-step launches, a and b in turn; the
+// last one writes the moments.  *in_b follows the launches that were made.
+template <typename T>
+int step_run_impl(T *a, T *b, int64_t nx, int64_t ny, int layout, T omega, int bc, T u0, int64_t runs,
+                  int multi_variant, int64_t single, int variant, T *rho, T *ux, T *uy, int *in_b,
+                  void *stream) {
+    if (!in_b) return LBM_E_NULL;
+    *in_b = 0;
+    if (runs < 0 || single < 0) return LBM_E_SIZE;
+    for (int64_t p = 0; p < runs + single; ++p) {
+        const bool last = p + 1 == runs + single;
+        const T *src = *in_b ? b : a;
+        T *dst = *in_b ? a : b;
+        T *r = last ? rho : nullptr, *u = last ? ux : nullptr, *v = last ? uy : nullptr;
+        const int rc = p < runs ? multi_impl<T>(src, dst, nx, ny, layout, omega, bc, u0, r, u, v, multi_variant, stream)
+                                : step_impl<T>(src, dst, nx, ny, layout, omega, bc, u0, r, u, v, variant, stream);
+        if (rc) return rc;
+        *in_b = !*in_b;
+    }
+    return LBM_OK;
+}
+
 inline int multi_shape_info(int variant, int *steps, int64_t *min_nx, int64_t *min_ny) {
     const int shape = variant < 0 ? kDefaultMultiShape : variant;
 #define LBM_INFO_MULTI(id, k, tr, tc, bs, nts) \
@@ -1372,6 +1394,20 @@ int lbm_step_multi_f32(const float *src, float *dst, int64_t nx, int64_t ny, int
                        float omega, int bc, float u0, float *rho, float *ux, float *uy,
                        int variant, void *stream) {
     return multi_impl(src, dst, nx, ny, layout, omega, bc, u0, rho, ux, uy, variant, stream);
+}
+
+int lbm_step_run_f64(double *a, double *b, int64_t nx, int64_t ny, int layout, double omega, int bc,
+                     double u0, int64_t runs, int multi_variant, int64_t single, int variant,
+                     double *rho, double *ux, double *uy, int *in_b, void *stream) {
+    return step_run_impl<double>(a, b, nx, ny, layout, omega, bc, u0, runs, multi_variant, single, variant,
+                                 rho, ux, uy, in_b, stream);
+}
+
+int lbm_step_run_f32(float *a, float *b, int64_t nx, int64_t ny, int layout, float omega, int bc,
+                     float u0, int64_t runs, int multi_variant, int64_t single, int variant,
+                     float *rho, float *ux, float *uy, int *in_b, void *stream) {
+    return step_run_impl<float>(a, b, nx, ny, layout, omega, bc, u0, runs, multi_variant, single, variant,
+                                rho, ux, uy, in_b, stream);
 }
 
 int lbm_relayout(const void *src, void *dst, int64_t nx, int64_t ny, int elem_bytes,

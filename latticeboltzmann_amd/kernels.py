@@ -221,6 +221,34 @@ def step_multi(src, dst, omega, bc=nat.BC_CAVITY, u0=0.1, moments=None, variant=
     return dst
 
 
+def step_run(a, b, omega, bc, u0, runs, multi_variant, single, variant, moments=None,
+             layout=nat.LAYOUT_SOA):
+    """``runs`` ``step_multi`` launches and then ``single`` ``step`` launches from
+    ``a``, using ``a`` and ``b`` in turn, issued by one native call; ``moments``
+    receive those of the last step.  Returns (current, other) buffer."""
+    import ctypes
+    nx, ny = _populations(a, "step", layout)
+    _require_device(b)
+    suf = _suffix(a, "step")
+    _same(a, b, "step")
+    if b.shape != a.shape:
+        raise ValueError("step: output must match the input")
+    rho = ux = uy = None
+    if moments is not None:
+        rho, ux, uy = moments
+        _require_device(rho, ux, uy)
+        for t in (rho, ux, uy):
+            _same(a, t, "step")
+            if t.shape != (nx, ny):
+                raise ValueError("step: moment arrays must have shape (nx, ny)")
+    in_b = ctypes.c_int()
+    nat.call("lbm_step_run_" + suf, nat.ptr(a), nat.ptr(b), nx, ny, int(layout), float(omega),
+             int(bc), float(u0), runs, -1 if multi_variant is None else int(multi_variant), single,
+             int(variant), nat.ptr(rho), nat.ptr(ux), nat.ptr(uy), ctypes.byref(in_b),
+             nat.stream_ptr())
+    return (b, a) if in_b.value else (a, b)
+
+
 class Workspace:
     """Device scratch of the two-pass reductions plus a device result slot."""
 

@@ -15,6 +15,7 @@ domain.
 """
 
 import math
+import operator
 
 import numpy as np
 import torch
@@ -156,19 +157,12 @@ class Lattice:
         """Advance ``n`` steps.  ``moments=(rho, ux, uy)`` tensors receive the
         pre-collision moments of the last step.  Runs of K steps go through the
         multi-step kernel when enabled; the bits are those of n single steps."""
-        bc = BCS[self.bc]
-        runs = self._runs(n)
-        single = n - runs * self.multi_k
-        for p in range(runs):
-            mom = moments if (moments is not None and p == runs - 1 and single == 0) else None
-            kernels.step_multi(self.f, self._g, self.omega, bc, self.u0, moments=mom,
-                               variant=self.multi_variant, layout=self.layout)
-            self.f, self._g = self._g, self.f
-        for s in range(single):
-            mom = moments if (moments is not None and s == single - 1) else None
-            kernels.step(self.f, self._g, self.omega, bc, self.u0, moments=mom,
-                         variant=self.variant, layout=self.layout)
-            self.f, self._g = self._g, self.f
+        n = operator.index(n)
+        if n > 0:
+            runs = self._runs(n)
+            self.f, self._g = kernels.step_run(self.f, self._g, self.omega, BCS[self.bc], self.u0,
+                                               runs, self.multi_variant, n - runs * self.multi_k,
+                                               self.variant, moments=moments, layout=self.layout)
         self.time += n
         return self
 
