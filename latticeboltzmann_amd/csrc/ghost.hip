@@ -48,6 +48,7 @@ constexpr int kGhostBlock = 512;
 struct GhostParams {
     int nx, ny;
     int nrules, pbc_mode, flags;
+    int reach;  // columns from the inlet / outlet within which its values can matter
     double omega, rho_in, rho_out;
     lbm_ghost_rule rules[LBM_GHOST_MAX_RULES];
 };
@@ -293,38 +294,17 @@ __device__ __forceinline__ T rule_value(const Gr &g, const GhostParams &p, const
     return v;
 }
 
-// Target rectangle of rule `lane` (lanes >= nrules: empty), one rule per lane,
-// so that testing rule r reads its rectangle with readlane instead of waiting
-// for a load.  Only used where the whole wave is active.
-struct RuleRects {
-    int x0, w, y0, h;
-};
-
-__device__ __forceinline__ RuleRects rule_rects(const GhostParams &p) {
-    const int lane = int(threadIdx.x & 63);
-    RuleRects q{0, 0, 0, 0};
-    if (lane < p.nrules) {
-        const lbm_ghost_rule &r = p.rules[lane];
-        q = RuleRects{r.x0, r.x1 - r.x0, r.y0, r.y1 - r.y0};
-    }
-    return q;
-}
-
-// The nine values of node (X, Y) after streaming and the rules (ascending, the
-// scripts' order).  Called with all lanes of the wave active and one x for all.
+// The nine values of node (x, y) after streaming and the rules (ascending, the
+// scripts' order).  x is the same for all lanes, so most rules end at a scalar
+// branch.
 template <bool Pbc, typename Gr, typename T = typename Gr::value_type>
 __device__ __forceinline__ void node_values(const Gr &g, const GhostParams &p, int x, int y, T h[9]) {
     load_g9<Pbc>(g, p, x, y, h);
-    const RuleRects q = rule_rects(p);
-    // rules whose columns hold x
-    for (unsigned m = unsigned(__ballot(unsigned(x - q.x0) < unsigned(q.w))); m; m &= m - 1) {
-        const int r = __builtin_ctz(m);
-        const int y0 = __builtin_amdgcn_readlane(q.y0, r), n = __builtin_amdgcn_readlane(q.h, r);
-        const bool hit = unsigned(y - y0) < unsigned(n);
-        if (__ballot(hit)) {
-            const lbm_ghost_rule &rule = p.rules[r];
-            if (hit) put(h, rule.ch, rule_value<Pbc>(g, p, rule, x, y));
-        }
+    for (int r = 0; r < p.nrules; ++r) {
+        const lbm_ghost_rule &rule = p.rules[r];
+        if (unsigned(x - rule.x0) < unsigned(rule.x1 - rule.x0) &&
+            unsigned(y - rule.y0) < unsigned(rule.y1 - rule.y0))
+            put(h, rule.ch, rule_value<Pbc>(g, p, rule, x, y));
     }
 }
 
@@ -343,18 +323,18 @@ __global__ __launch_bounds__(kGhostBlock) void k_ghost_step(const T *__restrict_
                                                        const GhostParams p, T *__restrict__ rho_out,
                                                        T *__restrict__ ux_out, T *__restrict__ uy_out) {
     const int x = blockIdx.y;
-    const int y1 = blockIdx.x * kGhostBlock + threadIdx.x;
-    if ((y1 & ~63) >= p.ny) return;   // whole waves reach the rule tests
-    const int y = min(y1, p.ny - 1);
+    const int y = blockIdx.x * kGhostBlock + threadIdx.x;
+    if (y >= p.ny) return;
     const Grid<T, Rows> g{src, p.nx, p.ny};
     T h[9];
     if (p.flags & LBM_GHOST_COLLIDE_ONLY) {
 #pragma unroll
         for (int i = 0; i < 9; ++i) h[i] = g.at(i, x, y);
+    } else if (Pbc && (x < p.reach || x >= p.nx - p.reach)) {
+        node_values<true>(g, p, x, y, h);
     } else {
-        node_values<Pbc>(g, p, x, y, h);
+        node_values<false>(g, p, x, y, h);
     }
-    if (y1 >= p.ny) return;
     T rho = T(0), ux = T(0), uy = T(0);
     if (!(p.flags & LBM_GHOST_NO_COLLIDE)) sf_collide<T>(h, T(p.omega), rho, ux, uy);
 #pragma unroll
@@ -824,7 +804,12 @@ int ghost_params(const T *src, const T *dst, int64_t nx, int64_t ny, int layout,
         const int rc = check_rules(rules, nrules, p.nx, p.ny);
         if (rc) return rc;
         p.nrules = nrules;
-        for (int r = 0; r < nrules; ++r) p.rules[r] = rules[r];
+        p.reach = 2;  // pulls from columns 0 and nx-1 reach 1 and nx-2
+        for (int r = 0; r < nrules; ++r) {
+            p.rules[r] = rules[r];
+            const int d = rules[r].dx < 0 ? -rules[r].dx : rules[r].dx;
+            if (d + 2 > p.reach) p.reach = d + 2;  // sources at x + dx, pulls from there
+        }
     }
     return LBM_OK;
 }

@@ -2,13 +2,15 @@
 // trained and evaluated on the GPU, plus the initializer that turns its
 // prediction into populations.
 //
-// Convolutions are 3x3, stride 1, zero padding, NHWC activations.  They run
-// as im2col + GEMM: cols[pixel][(dy*3+dx)*C + c] (BF16) times the weights
+// Convolutions are 3x3, stride 1, zero padding, NHWC activations: products of the
+// neighbourhoods cols[pixel][(dy*3+dx)*C + c] (BF16) with the weights
 // W[cout][(dy*3+dx)*C + c] (BF16), accumulated in FP32 by v_mfma_f32_16x16x32_bf16
-// (gfx950).  Backward: dW = dY^T cols (split-K over pixels with a fixed-order
-// reduction), dcols = dY W, dX = col2im(dcols) as a gather (no atomics), so
-// every result is deterministic.  Activations are kept in FP32 with a BF16
-// copy for the next GEMM; weights in FP32 (Adam) with a BF16 copy.
+// (gfx950).  k_conv3p (packed weights) and k_conv3 do the forward pass and the
+// data gradient where the input channels are a multiple of 32, k_wgrad the weight
+// gradient (split over pixels, the splits added in order), k_gemm with its
+// gathering loaders the rest; no atomics, so every result is deterministic.
+// For training, activations are kept in FP32 with a BF16 copy for the next
+// product; weights in FP32 (Adam) with a BF16 copy.
 //
 // No reference counterpart: the reference has no learned component.
 

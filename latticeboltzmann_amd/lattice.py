@@ -2,8 +2,9 @@
 
 This is the engine behind the reference's driver loops
 (``cavity_opt1.py:338-347``, ``shear_wave_opt1.py:170-174``): two population
-buffers ping-pong through the fused pull stream-collide kernel, one launch
-per step, on one stream.  By default the populations are kept in the
+buffers ping-pong through the fused pull stream-collide kernels, up to eight
+steps per launch, on one stream; one native call issues the launches of a
+``step``.  By default the populations are kept in the
 row-interleaved layout ``f[k][i][l]`` (nine channel segments of an x-row
 adjacent in HBM), which streams faster than the reference's ``f[i][k][l]``;
 ``populations()`` and ``load()`` convert to and from the reference layout,

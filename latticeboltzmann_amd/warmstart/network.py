@@ -1,10 +1,9 @@
 """Convolutional encoder-decoder of the warm start, on the project's HIP kernels.
 
 Every arithmetic step runs in ``liblbm_d2q9.so`` (``lbm_nn_*``): 3x3 same
-convolutions as BF16 MFMA GEMMs with FP32 accumulation whose tile loader
-gathers the shifted activations itself (no im2col matrix in memory: forward,
-weight gradient and data gradient), a fused bias/ReLU epilogue, 2x2 average
-pooling, nearest 2x upsampling, channel concatenation, their backward passes,
+convolutions as BF16 MFMA products with FP32 accumulation that read the shifted
+activations themselves (no im2col matrix in memory: forward, weight gradient
+and data gradient), a fused bias/ReLU epilogue, 2x2 average pooling, nearest 2x upsampling, channel concatenation, their backward passes,
 the MSE loss and Adam.  torch provides
 device memory only (no autograd, no torch arithmetic on the hot path).
 
