@@ -556,7 +556,7 @@ __device__ __forceinline__ uint4 load_channels(__amdgpu_buffer_rsrc_t r, unsigne
 }
 
 constexpr int kWgradPx = 128;
-constexpr int64_t WGRAD_BLOCKS = 3;
+constexpr int64_t WGRAD_BLOCKS = 3;  // blocks a CU: its LDS holds three (43.5 KB each)
 
 template <int MT>
 __global__ __launch_bounds__(256) void k_wgrad(WgradArgs a) {
@@ -1315,6 +1315,8 @@ static bool wgrad_direct(const void *x, const void *dy, int64_t P, int cin, int 
 static int run_conv(const ConvArgs &a, hipStream_t s) {
     // The largest tile that still gives every SIMD two waves: operands loaded per
     // MFMA fall with the tile, but a wave's 9 C / 32 steps are a serial chain.
+    // 16 x 32 x 32, 256 -> 128: 4 x 2 tiles 54 us, 4 x 4 (one wave a SIMD) 73; batch 1,
+    // 128 -> 128: 1 x 1 10.6 us, 2 x 2 19.8.
     const int64_t simds = 4 * int64_t(device_cus());
     auto waves = [&](int mt, int nt) {
         return int64_t((a.P + 16 * mt - 1) / (16 * mt)) * ((a.N + 16 * nt - 1) / (16 * nt));
