@@ -546,8 +546,10 @@ int lbm_ghost_step_f32(const float *src, float *dst, int64_t nx, int64_t ny, int
                        void *stream);
 /* `steps` full steps (flags 0) from buffer a, using a and b in turn and up to
  * four steps per launch; bitwise the same as that many lbm_ghost_step calls.
- * *in_b says which buffer ends up with the state; rho/ux/uy receive the moments
- * of the last step.  Arguments are checked as by lbm_ghost_step.               */
+ * *in_b says which buffer ends up with the state: b for an odd number of steps,
+ * a for an even one, as after that many single steps (so a captured run of an
+ * even number can be replayed).  rho/ux/uy receive the moments of the last step.
+ * Arguments are checked as by lbm_ghost_step.                                  */
 int lbm_ghost_run_f64(double *a, double *b, int64_t nx, int64_t ny, int layout, double omega,
                       const lbm_ghost_rule *rules, int nrules, const lbm_ghost_pbc *pbc,
                       int64_t steps, double *rho, double *ux, double *uy, int *in_b, void *stream);

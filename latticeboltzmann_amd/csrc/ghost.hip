@@ -1023,9 +1023,20 @@ int ghost_run(T *a, T *b, int64_t nx, int64_t ny, int layout, double omega, cons
             if (ghost_multi<T>(order[k], a, b, layout, p, w, kGhostMaxK, rho, ux, uy, s, true))
                 shape = order[k];
     }
+    // The state has to end where single-step launches would leave it (a graph that a
+    // program captures of an even number of steps reads the buffer it ends in), so
+    // their number is odd for an odd number of steps, even for an even one.  Large
+    // tiles: four steps a launch as long as the others get one each, because a
+    // single step is HBM-bound and cheap beside two or three on tiles (4098^2 FP64
+    // sliding lid, us a launch of 1, 2, 3, 4 steps: 445, 664, 640, 692; canal 425,
+    // 667, 814, 977).  Small tiles: as even as possible (102 x 52 canal, two steps
+    // 10.3 us, three 13.6, four 16.6, a single step 12.1).
+    int64_t launches = shape < 0 ? steps : (steps + kGhostMaxK - 1) / kGhostMaxK;
+    if ((launches ^ steps) & 1) ++launches;
     T *src = a, *dst = b;
-    while (steps > 0) {
-        const int K = shape < 0 ? 1 : int(steps < kGhostMaxK ? steps : kGhostMaxK);
+    for (; launches > 0; --launches) {
+        const int64_t most = shape == 2 ? (steps + launches - 1) / launches : steps - launches + 1;
+        const int K = int(most < kGhostMaxK ? most : kGhostMaxK);
         const bool last = steps == K;
         T *r = last ? rho : nullptr, *u = last ? ux : nullptr, *v = last ? uy : nullptr;
         if (K == 1) {

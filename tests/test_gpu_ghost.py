@@ -203,3 +203,41 @@ def test_several_steps_per_launch_match_oracle(gpu, flow, tdt, ndt, nx, ny, step
         after(G)
         omom = g.collide(G, 1.3)
     same(lat, mom, G, omom)
+
+
+@pytest.mark.parametrize("flow,nx,ny", [("lid", 45, 67), ("canal", 102, 52), ("poiseuille", 700, 500)])
+@pytest.mark.parametrize("steps", [1, 2, 4, 5, 10, 12, 20, 100])
+def test_step_ends_in_the_buffer_of_single_steps(gpu, flow, nx, ny, steps):
+    # n steps leave the state where n single-step launches would, so graphs of an
+    # even number of steps (StepGraph's, or captured by a program) can be replayed
+    from latticeboltzmann_amd import ghost
+    from latticeboltzmann_amd.lattice import StepGraph
+    rules = {"lid": lambda: ghost.cavity_walls(nx, ny, 0.1), "poiseuille": lambda: ghost.channel_walls(nx, ny, 0.02),
+             "canal": lambda: ghost.side_walls(nx, ny) + ghost.obstacle_faces(50, 24, 53, 27)}[flow]()
+    pbc = {"lid": None, "canal": ("after", 1.01, 0.99), "poiseuille": ("before", 1.01, 0.99)}[flow]
+    lat, ref = (ghost.GhostLattice(nx, ny, 1.3, rules, pbc) for _ in range(2))
+    print("buffers", flow, nx, ny, steps, flush=True)
+
+    def eager(n):
+        for _ in range(n):
+            ref.step(1)
+
+    a, b = lat.f, lat._g
+    lat.step(steps)
+    eager(steps)
+    assert lat.f.data_ptr() == (b if steps % 2 else a).data_ptr()
+    assert torch.equal(lat.f, ref.f)
+    with StepGraph(lat, steps) as advance:
+        for odd in (0, 1, 0, 3):  # replays, with eager work that moves the state in between
+            advance()
+            lat.step(odd)
+            eager(steps + odd)
+            assert torch.equal(lat.f, ref.f) and lat.time == ref.time
+
+
+@pytest.mark.parametrize("tdt,ndt", DT)
+@pytest.mark.parametrize("nx,ny,steps", [(45, 67, 8), (45, 67, 10), (361, 1067, 8), (352, 1058, 10)])
+@pytest.mark.parametrize("flow", ["lid", "poiseuille", "canal"])
+def test_launch_splits_match_oracle(gpu, flow, tdt, ndt, nx, ny, steps):
+    # launches of 4 + 4, 3 + 3 + 2 + 2 (small tiles) and 4 + 4 + 1 + 1 steps
+    test_several_steps_per_launch_match_oracle(gpu, flow, tdt, ndt, nx, ny, steps)
