@@ -48,10 +48,12 @@ _WALLS_IN_PLACE = 48 << 20
 
 def _plain(f):
     """A tensor whose memory the kernels may rewrite as it lies; the others
-    (views, autograd leaves, lazily conjugated or negated ones) go through a
-    second array and torch's own copy_ with its rules."""
+    (views, autograd leaves, lazily conjugated or negated ones, inference tensors
+    outside inference mode) go through a second array and torch's own copy_ with
+    its rules."""
     return (type(f) is torch.Tensor and f.is_contiguous() and not f.requires_grad
-            and not f.is_conj() and not f.is_neg())
+            and not f.is_conj() and not f.is_neg()
+            and (torch.is_inference_mode_enabled() or not f.is_inference()))
 
 
 def stream(f_ikl):

@@ -359,3 +359,24 @@ def test_streaming_in_place_equals_second_array(gpu, nx, ny):
     leaf = torch.rand((9, nx, ny), device="cuda", requires_grad=True)
     with pytest.raises(RuntimeError):
         PyLB.stream(leaf)
+
+
+@pytest.mark.parametrize("nx,ny", [(64, 64), (1024, 700)])
+def test_streaming_of_inference_tensors(gpu, nx, ny):
+    # writable inside inference mode, refused by copy_ outside it
+    from latticeboltzmann_amd import PyLB, kernels
+    with torch.inference_mode():
+        f = torch.rand((9, nx, ny), device="cuda", dtype=torch.float64)
+        for ref, call in ((kernels.stream(f), PyLB.stream),
+                          (kernels.stream_bounce_back(f, 0.1), PyLB.stream_and_bounce_back)):
+            g = f.clone()
+            call(g)
+            assert torch.equal(g, ref)
+    for call in (PyLB.stream, PyLB.stream_and_bounce_back):
+        with pytest.raises(RuntimeError):
+            call(f)
+    plain = torch.rand((9, nx, ny), device="cuda")  # an ordinary tensor in inference mode
+    with torch.inference_mode():
+        ref = kernels.stream(plain)
+        PyLB.stream(plain)
+        assert torch.equal(plain, ref)
