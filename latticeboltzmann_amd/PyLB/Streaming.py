@@ -18,6 +18,7 @@ tensors on a ROCm device are processed on the device.
 
 import numpy as np
 import torch
+from torch.autograd import forward_ad
 
 from latticeboltzmann_amd import kernels
 from . import _staging
@@ -49,11 +50,12 @@ _WALLS_IN_PLACE = 48 << 20
 def _plain(f):
     """A tensor whose memory the kernels may rewrite as it lies; the others
     (views, autograd leaves, lazily conjugated or negated ones, inference tensors
-    outside inference mode) go through a second array and torch's own copy_ with
-    its rules."""
+    outside inference mode, tensors with a forward-mode tangent) go through a
+    second array and torch's own copy_ with its rules."""
     return (type(f) is torch.Tensor and f.is_contiguous() and not f.requires_grad
             and not f.is_conj() and not f.is_neg()
-            and (torch.is_inference_mode_enabled() or not f.is_inference()))
+            and (torch.is_inference_mode_enabled() or not f.is_inference())
+            and forward_ad.unpack_dual(f).tangent is None)
 
 
 def stream(f_ikl):
