@@ -40,11 +40,33 @@ def _check_populations(f, name):
     return f.shape[1] > 0 and f.shape[2] > 0
 
 
-# The cavity form in place takes three launches, through a second array two: below
-# about 48 MB the launches count (64^2 FP64 18.4 us against 15.9, 43 MB 30.8 against
-# 29.8), above it the bytes (54 MB 31 against 37, 2048^2 FP64 114 against 232).  The
-# periodic form takes two either way.
-_WALLS_IN_PLACE = 48 << 20
+# Streaming in place moves half the bytes of a second array and a copy back, but a
+# thread moves one value at a time down 16 rows and one block shifts a whole row, so
+# it needs wide values, rows that fill their blocks, and rows enough to fill the GPU
+# or short enough to be quick.  us a call in place against the second array:
+#   1- and 2-byte values: uint8 3000 x 2000 57.6 / 41.8, FP16 6000 x 200 22.1 / 18.0
+#     (2048^2 42.9 / 47.4): second array;
+#   FP64 2048^2 105 / 235, FP32 2048^2 52 / 122, 1500 x 700 17.1 / 26.7;
+#   rows of 512 bytes, FP64 6000 x 64 16.8 / 19.3, FP32 6000 x 128 18.0 / 19.4; FP32
+#     6000 x 64 15.8 / 15.5, FP64 100000 x 10 186 / 73;
+#   few long rows: FP32 64 x 20000 40.5 / 30.7, FP64 3 x 500000 760 / 64, but FP32
+#     256 x 100000 644 / 687 and 64 x 6000 13.2 / 15.7.
+# Small arrays are bound by the host, where the second array costs less (512^2, a
+# call: FP32, 9.4 MB, 15.3 / 14.6, FP64 15.3 / 16.8).  The cavity form takes three
+# launches against two and its side walls touch a cache line per row: it wants 48 MB
+# (43 MB 30.8 / 29.8, 54 MB 31 / 37) and rows of 1024 bytes (FP64 100000 x 128
+# 557 / 708, FP32 100000 x 128 361 / 343).
+_IN_PLACE, _WALLS_IN_PLACE = 12 << 20, 48 << 20
+_ROW_BYTES, _WALLS_ROW_BYTES = 512, 1024
+_MANY_ROWS, _SHORT_ROW = 256, 6144
+
+
+def _in_place(f, walls):
+    if f.nbytes < (_WALLS_IN_PLACE if walls else _IN_PLACE):
+        return False
+    size, (_, nx, ny) = f.element_size(), f.shape
+    return (size >= 4 and (nx >= _MANY_ROWS or ny <= _SHORT_ROW)
+            and ny * size >= (_WALLS_ROW_BYTES if walls else _ROW_BYTES) and _plain(f))
 
 
 def _plain(f):
@@ -68,7 +90,7 @@ def stream(f_ikl):
     if isinstance(f_ikl, np.ndarray):
         out = kernels.stream(_staging.to_device(f_ikl))
         _staging.write_back(f_ikl, out)
-    elif _plain(f_ikl):
+    elif _in_place(f_ikl, False):
         kernels.stream_in_place(f_ikl)
         _staging.written(f_ikl)
     else:
@@ -90,7 +112,7 @@ def stream_and_bounce_back(f_ikl, u0=0.1):
     if isinstance(f_ikl, np.ndarray):
         out = kernels.stream_bounce_back(_staging.to_device(f_ikl), float(u0))
         _staging.write_back(f_ikl, out)
-    elif _plain(f_ikl) and f_ikl.numel() * f_ikl.element_size() >= _WALLS_IN_PLACE:
+    elif _in_place(f_ikl, True):
         kernels.stream_in_place(f_ikl, float(u0))
         _staging.written(f_ikl)
     else:

@@ -396,3 +396,15 @@ def test_streaming_of_forward_mode_tensors(gpu):
                 primal, tangent = fwd.unpack_dual(d)
                 assert torch.equal(primal, ref)
                 assert tangent is None or not tangent.any()
+
+
+@pytest.mark.parametrize("nx,ny", [(1, 1), (1, 7), (7, 1), (2, 2), (3, 5), (17, 33), (32, 257), (33, 300),
+                                   (40, 2049), (5, 4101), (1000, 130)])
+def test_streaming_in_place_kernels_at_any_size(gpu, nx, ny):
+    # also where PyLB.stream takes a second array
+    from latticeboltzmann_amd import kernels
+    gen = torch.Generator(device="cuda").manual_seed(nx * 7 + ny)
+    for dt in (torch.uint8, torch.int16, torch.float32, torch.float64):
+        f = torch.randint(0, 250, (9, nx, ny), device="cuda", generator=gen).to(dt)
+        ref = kernels.stream(f)
+        assert torch.equal(kernels.stream_in_place(f), ref), dt
