@@ -65,7 +65,8 @@ def _in_place(f, walls):
     if f.nbytes < (_WALLS_IN_PLACE if walls else _IN_PLACE):
         return False
     size, (_, nx, ny) = f.element_size(), f.shape
-    return (size >= 4 and (nx >= _MANY_ROWS or ny <= _SHORT_ROW)
+    # blocks of 256 threads of a launch, at most: 2.4 a row segment of 256 values
+    return (size >= 4 and (nx >= _MANY_ROWS or ny <= _SHORT_ROW) and 3 * nx * (ny // 256 + 1) < 1 << 24
             and ny * size >= (_WALLS_ROW_BYTES if walls else _ROW_BYTES) and _plain(f))
 
 

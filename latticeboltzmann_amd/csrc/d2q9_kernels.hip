@@ -1156,16 +1156,31 @@ int stream_bounce_impl(const T *src, T *dst, int64_t nx, int64_t ny, T u0, void 
     return launch_status();
 }
 
+// Blocks of k_inplace_save and k_inplace_move; a launch takes fewer than 2^32 threads,
+// which rows of one segment reach at 7 million rows (a pass into a second array,
+// one block a row segment, at 16.7 million).
+struct InplaceGrid {
+    int64_t nb, nseg, chains, cols;
+    InplaceGrid(int64_t nx, int64_t ny, bool walls)
+        : nb((nx + kInRows - 1) / kInRows), nseg((ny + kBlock - 1) / kBlock), chains(nb * 6 * nseg),
+          cols(walls ? (nx + kBlock - 1) / kBlock : 0) {}
+    bool fits(int64_t nx) const {
+        const int64_t most = (int64_t(1) << 32) / kBlock - 1;
+        return chains + cols <= most && chains + 2 * nx <= most;
+    }
+};
+
 inline int64_t inplace_scratch(int64_t nx, int64_t ny, bool walls) {
-    return (nx + kInRows - 1) / kInRows * 6 * ny + (walls ? 6 * nx : 0);
+    const InplaceGrid g(nx, ny, walls);
+    if (!g.fits(nx)) return LBM_E_SIZE;
+    return g.nb * 6 * ny + (walls ? 6 * nx : 0);
 }
 
 template <typename U, bool Walls>
 int launch_inplace(U *f, U *scratch, int64_t nx, int64_t ny, U u0, hipStream_t s) {
-    const int64_t nb = (nx + kInRows - 1) / kInRows, nseg = (ny + kBlock - 1) / kBlock;
-    const int64_t chains = nb * 6 * nseg, cols = Walls ? (nx + kBlock - 1) / kBlock : 0;
-    if (nx > 0x3fffffff || ny > 0x3fffffff || chains + cols > 0x7fffffffLL || chains + 2 * nx > 0x7fffffffLL)
-        return LBM_E_SIZE;
+    const InplaceGrid g(nx, ny, Walls);
+    if (!g.fits(nx)) return LBM_E_SIZE;
+    const int64_t nb = g.nb, nseg = g.nseg, chains = g.chains, cols = g.cols;
     hipLaunchKernelGGL((k_inplace_save<U, Walls>), dim3(unsigned(chains + cols)), dim3(kBlock), 0, s, f,
                        scratch, int(nx), int(ny), int(nb), int(nseg), chains);
     hipLaunchKernelGGL(k_inplace_move<U>, dim3(unsigned(chains + 2 * nx)), dim3(kBlock), 0, s, f, scratch,

@@ -164,3 +164,23 @@ def test_streaming_route(dtype, nx, ny, periodic, walls):
     f = torch.empty((9, nx, ny), dtype=dtype, device="meta")
     assert Streaming._in_place(f, False) == periodic
     assert Streaming._in_place(f, True) == walls
+
+
+def test_streaming_route_beyond_one_launch():
+    # grids that take more than 2^32 threads in place go through a second array,
+    # which takes fewer; the in-place calls say so before any launch
+    from latticeboltzmann_amd import _native as nat
+    from latticeboltzmann_amd.PyLB import Streaming
+    lib = nat.load()
+    for nx, fits in ((5 << 20, True), (8 << 20, False)):
+        f = torch.empty((9, nx, 128), dtype=torch.float32, device="meta")
+        assert Streaming._in_place(f, False) == fits
+        assert (lib.lbm_stream_inplace_scratch(nx, 128, 0) > 0) == fits
+        assert (lib.lbm_stream_inplace_scratch(nx, 128, 1) > 0) == fits
+    assert lib.lbm_stream_inplace_scratch(8 << 20, 128, 0) == -2
+    # every grid that the route takes fits
+    for nx in (1, 255, 256, 5000, 1 << 20, 5592405, 1 << 23, 1 << 24):
+        for ny in (128, 255, 256, 1000, 6144, 6145, 1 << 20, 1 << 26):
+            f = torch.empty((9, nx, ny), dtype=torch.float64, device="meta")
+            for walls in (False, True):
+                assert not Streaming._in_place(f, walls) or lib.lbm_stream_inplace_scratch(nx, ny, walls) > 0
