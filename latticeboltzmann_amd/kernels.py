@@ -10,6 +10,8 @@ in one of two layouts:
   x-row adjacent (the layout the device-resident solver keeps in HBM).
 """
 
+import ctypes
+
 import torch
 
 from . import _native as nat
@@ -222,11 +224,12 @@ def step_multi(src, dst, omega, bc=nat.BC_CAVITY, u0=0.1, moments=None, variant=
 
 
 def step_run(a, b, omega, bc, u0, runs, multi_variant, single, variant, moments=None,
-             layout=nat.LAYOUT_SOA):
+             layout=nat.LAYOUT_SOA, in_b=None):
     """``runs`` ``step_multi`` launches and then ``single`` ``step`` launches from
     ``a``, using ``a`` and ``b`` in turn, issued by one native call; ``moments``
-    receive those of the last step.  Returns (current, other) buffer."""
-    import ctypes
+    receive those of the last step.  Returns (current, other) buffer.  ``in_b`` (a
+    ``ctypes.c_int`` of 0) is set to 1, also when the call raises, if the launches
+    made have left the state in ``b``."""
     nx, ny = _populations(a, "step", layout)
     _require_device(b)
     suf = _suffix(a, "step")
@@ -241,7 +244,8 @@ def step_run(a, b, omega, bc, u0, runs, multi_variant, single, variant, moments=
             _same(a, t, "step")
             if t.shape != (nx, ny):
                 raise ValueError("step: moment arrays must have shape (nx, ny)")
-    in_b = ctypes.c_int()
+    if in_b is None:
+        in_b = ctypes.c_int()
     nat.call("lbm_step_run_" + suf, nat.ptr(a), nat.ptr(b), nx, ny, int(layout), float(omega),
              int(bc), float(u0), runs, -1 if multi_variant is None else int(multi_variant), single,
              int(variant), nat.ptr(rho), nat.ptr(ux), nat.ptr(uy), ctypes.byref(in_b),

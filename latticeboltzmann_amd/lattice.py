@@ -15,6 +15,7 @@ The MPI decomposition and halo exchange of the reference
 domain.
 """
 
+import ctypes
 import math
 import operator
 
@@ -161,9 +162,14 @@ class Lattice:
         n = operator.index(n)
         if n > 0:
             runs = self._runs(n)
-            self.f, self._g = kernels.step_run(self.f, self._g, self.omega, BCS[self.bc], self.u0,
-                                               runs, self.multi_variant, n - runs * self.multi_k,
-                                               self.variant, moments=moments, layout=self.layout)
+            in_b = ctypes.c_int()
+            try:
+                kernels.step_run(self.f, self._g, self.omega, BCS[self.bc], self.u0, runs,
+                                 self.multi_variant, n - runs * self.multi_k, self.variant,
+                                 moments=moments, layout=self.layout, in_b=in_b)
+            finally:  # a launch that fails leaves the state of those before it
+                if in_b.value:
+                    self.f, self._g = self._g, self.f
         self.time += n
         return self
 

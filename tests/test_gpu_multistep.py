@@ -190,3 +190,21 @@ def test_small_grid_defaults_equal_single_steps(gpu, dtype, nx, ny):
         one.step(n, moments=m1)
         assert torch.equal(lat.f, one.f)
         assert all(torch.equal(a, b) for a, b in zip(m, m1))
+
+
+@pytest.mark.parametrize("n,done", [(1, 0), (9, 8), (13, 12), (17, 16)])
+def test_refused_step_leaves_the_steps_before_it(gpu, n, done):
+    # the single steps left over from the multi-step launches are refused
+    from latticeboltzmann_amd.lattice import Lattice
+    f = populations(64, 64, torch.float64)
+    lat = Lattice(64, 64, 1.3, "cavity", 0.1).load(f)
+    ref = Lattice(64, 64, 1.3, "cavity", 0.1, multi_step=False).load(f)
+    lat.variant = 10 ** 6
+    with pytest.raises(ValueError):
+        lat.step(n)
+    ref.step(done)
+    assert torch.equal(lat.f, ref.f) and lat.time == 0
+    lat.variant = -1
+    lat.step(5)
+    ref.step(5)
+    assert torch.equal(lat.f, ref.f)

@@ -184,3 +184,28 @@ def test_streaming_route_beyond_one_launch():
             f = torch.empty((9, nx, ny), dtype=torch.float64, device="meta")
             for walls in (False, True):
                 assert not Streaming._in_place(f, walls) or lib.lbm_stream_inplace_scratch(nx, ny, walls) > 0
+
+
+class _FailingRun:
+    """Stands for the native library: its run makes an odd number of launches,
+    then fails."""
+
+    def call(self, name, *args):
+        assert "_run_" in name
+        args[-2]._obj.value = 1
+        raise RuntimeError("HIP error")
+
+
+def test_failed_lattice_run_leaves_the_state_of_its_launches(monkeypatch):
+    from latticeboltzmann_amd import _native as nat
+    from latticeboltzmann_amd import kernels
+    from latticeboltzmann_amd.lattice import Lattice
+    monkeypatch.setattr(nat, "call", _FailingRun().call)
+    monkeypatch.setattr(nat, "stream_ptr", lambda: 0)
+    monkeypatch.setattr(kernels, "_require_device", lambda *t: None)
+    a, b = (torch.zeros((64, 9, 64), dtype=torch.float64) for _ in range(2))
+    lat = _bare(Lattice, f=a, _g=b, omega=1.2, bc="cavity", u0=0.1, layout=nat.LAYOUT_ROWS, variant=-1,
+                multi_variant=None, multi_k=1, time=0)
+    with pytest.raises(RuntimeError):
+        lat.step(3)
+    assert lat.f is b and lat._g is a and lat.time == 0
