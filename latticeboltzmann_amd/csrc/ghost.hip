@@ -1007,6 +1007,7 @@ int ghost_run(T *a, T *b, int64_t nx, int64_t ny, int layout, double omega, cons
               int nrules, const lbm_ghost_pbc *pbc, int64_t steps, T *rho, T *ux, T *uy, int *in_b,
               void *stream) {
     if (!in_b) return LBM_E_NULL;
+    *in_b = 0;
     GhostParams p;
     int rc = ghost_params<T>(a, b, nx, ny, layout, omega, rules, nrules, pbc, 0, rho, ux, uy, p);
     if (rc) return rc;
@@ -1033,8 +1034,9 @@ int ghost_run(T *a, T *b, int64_t nx, int64_t ny, int layout, double omega, cons
     // 10.3 us, three 13.6, four 16.6, a single step 12.1).
     int64_t launches = shape < 0 ? steps : (steps + kGhostMaxK - 1) / kGhostMaxK;
     if ((launches ^ steps) & 1) ++launches;
-    T *src = a, *dst = b;
     for (; launches > 0; --launches) {
+        const T *src = *in_b ? b : a;
+        T *dst = *in_b ? a : b;
         const int64_t most = shape == 2 ? (steps + launches - 1) / launches : steps - launches + 1;
         const int K = int(most < kGhostMaxK ? most : kGhostMaxK);
         const bool last = steps == K;
@@ -1046,12 +1048,9 @@ int ghost_run(T *a, T *b, int64_t nx, int64_t ny, int layout, double omega, cons
             rc = launch_status();
         }
         if (rc) return rc;
-        T *t = src;
-        src = dst;
-        dst = t;
+        *in_b = !*in_b;
         steps -= K;
     }
-    *in_b = src == b;
     return LBM_OK;
 }
 

@@ -249,13 +249,16 @@ class GhostLattice:
         if n > 0:
             rho, ux, uy = moments if moments is not None else (None, None, None)
             in_b = ctypes.c_int()
-            nat.call("lbm_ghost_run_" + _SUFFIX[self.dtype], nat.ptr(self.f), nat.ptr(self._g),
-                     self.nx, self.ny, self.layout, self.omega, ctypes.addressof(self._rules),
-                     len(self.rules),
-                     ctypes.addressof(self._pbc) if self._pbc is not None else None, n,
-                     nat.ptr(rho), nat.ptr(ux), nat.ptr(uy), ctypes.byref(in_b), nat.stream_ptr())
-            if in_b.value:
-                self.f, self._g = self._g, self.f
+            try:
+                nat.call("lbm_ghost_run_" + _SUFFIX[self.dtype], nat.ptr(self.f), nat.ptr(self._g),
+                         self.nx, self.ny, self.layout, self.omega, ctypes.addressof(self._rules),
+                         len(self.rules),
+                         ctypes.addressof(self._pbc) if self._pbc is not None else None, n,
+                         nat.ptr(rho), nat.ptr(ux), nat.ptr(uy), ctypes.byref(in_b),
+                         nat.stream_ptr())
+            finally:  # a launch that fails leaves the state of those before it
+                if in_b.value:
+                    self.f, self._g = self._g, self.f
         self.time += n
         return self
 

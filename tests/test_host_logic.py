@@ -209,3 +209,27 @@ def test_failed_lattice_run_leaves_the_state_of_its_launches(monkeypatch):
     with pytest.raises(RuntimeError):
         lat.step(3)
     assert lat.f is b and lat._g is a and lat.time == 0
+
+
+def test_failed_ghost_run_leaves_the_state_of_its_launches(monkeypatch):
+    from latticeboltzmann_amd import _native as nat
+    from latticeboltzmann_amd.ghost import GhostLattice
+    monkeypatch.setattr(nat, "call", _FailingRun().call)
+    monkeypatch.setattr(nat, "stream_ptr", lambda: 0)
+    a, b = (torch.zeros((30, 9, 40), dtype=torch.float64) for _ in range(2))
+    lat = _bare(GhostLattice, f=a, _g=b, nx=30, ny=40, omega=1.2, layout=nat.LAYOUT_ROWS, rules=[],
+                _rules=(nat.GhostRule * 1)(), _pbc=None, dtype=torch.float64, time=0)
+    with pytest.raises(RuntimeError):
+        lat.step(3)
+    assert lat.f is b and lat._g is a and lat.time == 0
+
+
+def test_native_ghost_run_says_where_the_state_is():
+    # *in_b is 0 when a run is refused before its first launch, whatever it held
+    from latticeboltzmann_amd import _native as nat
+    lib = nat.load()
+    for nx, steps, status in ((2, 3, -2), (30, -1, -2)):
+        in_b = ctypes.c_int(7)
+        assert lib.lbm_ghost_run_f64(1 << 20, 1 << 30, nx, 40, 0, 1.2, None, 0, None, steps, None, None, None,
+                                     ctypes.byref(in_b), None) == status
+        assert in_b.value == 0
