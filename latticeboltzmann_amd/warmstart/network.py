@@ -59,18 +59,7 @@ class Surrogate:
             self.offsets[name] = (n, n + 9 * cin * cout)
             n += 9 * cin * cout + cout
         self.nparams = n
-        # tables of the native calls: widths; weight offsets, channels and packed
-        # places of every layer
-        k = len(self.layers)
-        self._widths = (ctypes.c_int * len(self.widths))(*self.widths)
-        self._from = (ctypes.c_int64 * k)(*(self.offsets[l[0]][0] for l in self.layers))
-        self._cin = (ctypes.c_int * k)(*(l[1] for l in self.layers))
-        self._cout = (ctypes.c_int * k)(*(l[2] for l in self.layers))
-        self._to, self.packed, size = (ctypes.c_int64 * k)(), {}, 0
-        for i, (name, cin, cout, _) in enumerate(self.layers):
-            self._to[i] = self.packed[name] = size
-            size += int(nat.load().lbm_nn_packed_size(cin, cout))
-        self._packed_size = size
+        self._make_tables()
         f32 = dict(dtype=torch.float32, device=self.device)
         self.p = torch.empty(n, **f32)
         self.pb = torch.empty(n, dtype=torch.bfloat16, device=self.device)
@@ -82,6 +71,30 @@ class Surrogate:
         self.work = torch.empty(int(nat.load().lbm_reduce_workspace_bytes()) // 8,
                                 dtype=torch.float64, device=self.device)
         self.init_params(seed)
+
+    # Tables of the native calls: widths; weight offsets, channels and packed places
+    # of every layer.  ctypes arrays cannot be pickled: a pickled network leaves them
+    # out and makes them anew.
+    _TABLES = ("_widths", "_from", "_cin", "_cout", "_to", "packed", "_packed_size")
+
+    def _make_tables(self):
+        k = len(self.layers)
+        self._widths = (ctypes.c_int * len(self.widths))(*self.widths)
+        self._from = (ctypes.c_int64 * k)(*(self.offsets[l[0]][0] for l in self.layers))
+        self._cin = (ctypes.c_int * k)(*(l[1] for l in self.layers))
+        self._cout = (ctypes.c_int * k)(*(l[2] for l in self.layers))
+        self._to, self.packed, size = (ctypes.c_int64 * k)(), {}, 0
+        for i, (name, cin, cout, _) in enumerate(self.layers):
+            self._to[i] = self.packed[name] = size
+            size += int(nat.load().lbm_nn_packed_size(cin, cout))
+        self._packed_size = size
+
+    def __getstate__(self):
+        return {k: v for k, v in self.__dict__.items() if k not in self._TABLES}
+
+    def __setstate__(self, state):
+        self.__dict__.update(state)
+        self._make_tables()
 
     # -- parameters -------------------------------------------------------------
     def init_params(self, seed=0):

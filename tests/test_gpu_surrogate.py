@@ -585,3 +585,31 @@ def test_native_forward_equals_kept_forward(gpu, in_ch, widths, mid, B, H, W):
     assert torch.equal(net.forward(x), again) and not torch.equal(again, kept)
     lib = _nat().load()
     assert lib.lbm_nn_unet_workspace(1, 5, 8, 4, None, 1, 8, 3) == -2
+
+
+def test_networks_can_be_pickled_and_copied(gpu):
+    import copy
+    import io
+    import pickle
+
+    from latticeboltzmann_amd.warmstart.network import Surrogate
+    net = Surrogate(in_ch=5, widths=(32, 40), mid=24, seed=2)
+    x = torch.randn(2, 12, 20, 5, device="cuda", generator=torch.Generator("cuda").manual_seed(1))
+    t = torch.randn(2, 12, 20, 3, device="cuda", generator=torch.Generator("cuda").manual_seed(2))
+    net.train_step(x, t, 1e-4)
+    out = net.forward(x)
+    buf = io.BytesIO()
+    torch.save(net, buf)  # written here, so it may be unpickled
+    buf.seek(0)
+    # a state without the tables of the native calls, as a pickle of before them holds
+    state = {k: net.__dict__[k] for k in ("in_ch", "widths", "mid", "out_ch", "layers", "spec", "device", "offsets",
+                                          "nparams", "p", "pb", "g", "m", "v", "step_count", "ema", "work")}
+    old = Surrogate.__new__(Surrogate)
+    old.__setstate__(copy.deepcopy(state))
+    others = [pickle.loads(pickle.dumps(net)), copy.deepcopy(net), torch.load(buf, weights_only=False), old]
+    for other in others:
+        assert torch.equal(other.forward(x), out)
+    net.train_step(x, t, 1e-4)
+    for other in others:
+        other.train_step(x, t, 1e-4)
+        assert torch.equal(other.p, net.p) and torch.equal(other.forward(x), net.forward(x))
