@@ -1339,9 +1339,15 @@ static int64_t conv_lds(const ConvArgs &a, int mt) {
 }
 constexpr int64_t kConvLds = 80 * 1024;
 
+// Elements of the packed weights of K summed and N output channels; 0 where the
+// packed kernels do not apply (their offsets end at 2^31 bytes).
+static int64_t packed_elements(int K, int N) {
+    const int64_t n = K % 32 ? 0 : (int64_t(N) + 15) / 16 * 16 * 9 * K;
+    return n < (int64_t(1) << 30) ? n : 0;
+}
+
 static bool conv_packed_fits(const ConvArgs &a) {
-    const int64_t step_bytes = (int64_t(a.N) + 15) / 16 * (9 * a.C / 32) * 1024;
-    return conv_direct(a) && conv_lds(a, 1) <= kConvLds && step_bytes < (int64_t(1) << 31);
+    return conv_direct(a) && conv_lds(a, 1) <= kConvLds && packed_elements(a.C, a.N) > 0;
 }
 
 template <int MT, int NT, int D>
@@ -1384,9 +1390,7 @@ int lbm_nn_packed_fits(int B, int H, int W, int cin, int cout) {
 
 int64_t lbm_nn_packed_size(int cin, int cout) {
     if (cin <= 0 || cout <= 0) return LBM_E_SIZE;
-    // either orientation; 0 where the packed kernels do not apply
-    const int64_t f = cin % 32 ? 0 : (int64_t(cout) + 15) / 16 * 16 * 9 * cin;
-    const int64_t t = cout % 32 ? 0 : (int64_t(cin) + 15) / 16 * 16 * 9 * cout;
+    const int64_t f = packed_elements(cin, cout), t = packed_elements(cout, cin);  // either orientation
     return f > t ? f : t;
 }
 
@@ -1398,10 +1402,10 @@ int lbm_nn_pack_weights(const void *w, const int64_t *from, const int *cin, cons
     PackTable q{};
     q.transposed = transposed;
     for (int i = 0; i < n; ++i) {
-        if (cin[i] <= 0 || cout[i] <= 0 || int64_t(cin[i]) * cout[i] > (int64_t(1) << 26)) return LBM_E_SIZE;
+        if (cin[i] <= 0 || cout[i] <= 0) return LBM_E_SIZE;
         if (from[i] < 0 || to[i] < 0 || to[i] % 8) return LBM_E_ARG;
         const int K = transposed ? cout[i] : cin[i], N = transposed ? cin[i] : cout[i];
-        if (K % 32) continue;
+        if (!packed_elements(K, N)) continue;
         const int j = q.n++;
         q.from[j] = from[i], q.to[j] = to[i], q.cin[j] = cin[i], q.cout[j] = cout[i];
         q.first[j + 1] = q.first[j] + ((N + 15) / 16 * (9 * K / 32) * 64 + 255) / 256;
@@ -1444,7 +1448,7 @@ bool plan_unet(Unet &u, int B, int H, int W, int in_ch, const int *widths, int l
     auto add = [&](int cin, int cout, int level) {
         u.layer[u.n++] = Unet::Layer{cin, cout, level, flat, u.packed};
         flat += int64_t(9) * cin * cout + cout;
-        if (cin % 32 == 0) u.packed += (int64_t(cout) + 15) / 16 * 16 * 9 * cin;
+        u.packed += packed_elements(cin, cout);
     };
     int c = in_ch;
     for (int i = 0; i < levels; ++i) add(c, widths[i], i), add(widths[i], widths[i], i), c = widths[i];

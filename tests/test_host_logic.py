@@ -233,3 +233,24 @@ def test_native_ghost_run_says_where_the_state_is():
         assert lib.lbm_ghost_run_f64(1 << 20, 1 << 30, nx, 40, 0, 1.2, None, 0, None, steps, None, None, None,
                                      ctypes.byref(in_b), None) == status
         assert in_b.value == 0
+
+
+@pytest.mark.parametrize("cin,cout,transposed", [(16384, 8192, 0), (8192, 16384, 1), (65536, 2048, 0)])
+def test_packing_leaves_out_layers_beyond_the_packed_kernels(cin, cout, transposed):
+    # weights past 2^31 packed bytes run unpacked: no packed place, and packing a
+    # network that has such a layer is no error
+    from latticeboltzmann_amd import _native as nat
+    lib = nat.load()
+    assert lib.lbm_nn_packed_size(cin, cout) == 0
+    assert lib.lbm_nn_packed_fits(1, 2, 2, cin, cout) == 0
+    frm, to = (ctypes.c_int64 * 1)(0), (ctypes.c_int64 * 1)(0)
+    ci, co = (ctypes.c_int * 1)(cin), (ctypes.c_int * 1)(cout)
+    # nothing is launched, so no pointer is read
+    assert lib.lbm_nn_pack_weights(1 << 20, ctypes.addressof(frm), ctypes.addressof(ci), ctypes.addressof(co), 1,
+                                   transposed, 1 << 20, ctypes.addressof(to), None) == 0
+    assert lib.lbm_nn_packed_size(8192, 8192) == 9 * 8192 * 8192
+    # a network of such layers has a workspace without room for their packed weights
+    widths = (ctypes.c_int * 1)(32)
+    small = lib.lbm_nn_unet_workspace(1, 2, 2, 32, ctypes.addressof(widths), 1, 32, 3)
+    large = lib.lbm_nn_unet_workspace(1, 2, 2, 32, ctypes.addressof(widths), 1, 16384, 3)
+    assert 0 < small < large < small + (1 << 25)
