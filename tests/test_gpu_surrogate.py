@@ -613,3 +613,57 @@ def test_networks_can_be_pickled_and_copied(gpu):
     for other in others:
         other.train_step(x, t, 1e-4)
         assert torch.equal(other.p, net.p) and torch.equal(other.forward(x), net.forward(x))
+
+
+def _gemm_conv(nat, x, w, B, H, W, C, N, bias, relu):
+    """The convolution as im2col and a general GEMM: (FP32, BF16) outputs."""
+    P, K, sp = B * H * W, 9 * C, nat.stream_ptr()
+    cols = torch.empty((P, K), dtype=torch.bfloat16, device="cuda")
+    nat.call("lbm_nn_im2col3x3", _p(x), B, H, W, C, _p(cols), sp)
+    y, yb = (torch.empty((P, N), dtype=t, device="cuda") for t in (torch.float32, torch.bfloat16))
+    nat.call("lbm_nn_gemm", _p(cols), K, 1, _p(w), 1, K, _p(y), _p(yb), N, _p(bias), P, N, K, 0, relu, 1, None, sp)
+    return y, yb
+
+
+def _gemm_dgrad(nat, dy, w, B, H, W, C, N):
+    """The data gradient (C summed, N computed channels) on flipped weights and the
+    general GEMM, added to 0.25."""
+    sp = nat.stream_ptr()
+    wf = torch.empty(9 * C * N, dtype=torch.bfloat16, device="cuda")
+    nat.call("lbm_nn_conv3x3_flip_weights", _p(w), N, C, _p(wf), sp)
+    dx = torch.full((B * H * W, N), 0.25, device="cuda")
+    nat.call("lbm_nn_conv3x3_dgrad", _p(dy), _p(wf), B, H, W, N, C, _p(dx), 1, sp)
+    return dx
+
+
+# the block shapes of the direct kernel, 16 MT pixels x 16 NT channels a wave, each
+# with pixels and channels that do not fill the last one
+@pytest.mark.parametrize("tile,B,H,W,C,N", [((4, 4), 7, 139, 137, 32, 50), ((4, 4), 5, 100, 151, 64, 100),
+                                            ((4, 2), 5, 95, 99, 32, 90), ((4, 2), 7, 139, 137, 32, 18),
+                                            ((2, 2), 3, 101, 107, 32, 70), ((2, 2), 2, 150, 151, 96, 33),
+                                            ((1, 1), 3, 101, 107, 32, 3), ((1, 1), 2, 16, 20, 64, 18)])
+def test_direct_convolution_block_shapes(gpu, tile, B, H, W, C, N):
+    nat = _nat()
+    simds = 4 * torch.cuda.get_device_properties(0).multi_processor_count
+    P, sp = B * H * W, nat.stream_ptr()
+    chosen = (1, 1)  # the largest shape that gives every SIMD two waves
+    for mt, nt, over in ((4, 4, 32), (4, 2, 16), (2, 2, 16)):
+        if N > over and -(-P // (16 * mt)) * -(-N // (16 * nt)) >= 2 * simds:
+            chosen = (mt, nt)
+            break
+    print("direct", tile, chosen, B, H, W, C, N, flush=True)
+    assert chosen == tile or simds != 1024
+    rng = np.random.default_rng(C + N)
+    x, _ = _bf(rng, (B, H, W, C))
+    w, _ = _bf(rng, (N, 3, 3, C), 0.2)
+    bias = torch.as_tensor(rng.normal(size=N).astype(np.float32)).cuda()
+    ye, yeb = _gemm_conv(nat, x, w, B, H, W, C, N, bias, 1)
+    y, yb = torch.full_like(ye, float("nan")), torch.full_like(yeb, float("nan"))
+    nat.call("lbm_nn_conv3x3", _p(x), B, H, W, C, _p(w), N, _p(bias), _p(y), _p(yb), 1, sp)
+    assert torch.equal(y, ye) and torch.equal(yb, yeb)
+    w, _ = _bf(rng, (C, 3, 3, N), 0.2)  # a layer of N input channels, x its output's gradient
+    wt = torch.empty(9 * C * N, dtype=torch.bfloat16, device="cuda")
+    nat.call("lbm_nn_conv3x3_transpose_weights", _p(w), N, C, _p(wt), sp)
+    dx = torch.full((P, N), 0.25, device="cuda")
+    nat.call("lbm_nn_conv3x3_dgrad_t", _p(x), _p(wt), B, H, W, N, C, _p(dx), 1, sp)
+    assert torch.equal(dx, _gemm_dgrad(nat, x, w, B, H, W, C, N))
