@@ -1346,8 +1346,31 @@ static int64_t packed_elements(int K, int N) {
     return n < (int64_t(1) << 30) ? n : 0;
 }
 
-static bool conv_packed_fits(const ConvArgs &a) {
-    return conv_direct(a) && conv_lds(a, 1) <= kConvLds && packed_elements(a.C, a.N) > 0;
+// The block of k_conv3p for a layer, 32 MT pixels x 32 NT channels as 10 MT + NT; 0
+// where k_conv3 runs it.  us of layers (batch x side^2), and of k_conv3:
+//   41, 128 x 32, where 64 channels would leave half of the last block's waves
+//     without any (32 at most, or 65 to 96), from 3 blocks per two CUs.  32 -> 32 at
+//     4 x 112^2 9.0 (22: 9.4, k_conv3 10.8), 3 x 128^2 9.1 (8.7, 9.8), 16 x 128^2
+//     25.7 (30.0, 25.0); 96 -> 32 at 4 x 112^2 12.7 (22.0, 26.8), 8 x 128^2 32.9
+//     (53.8, 31.7), 16 x 128^2 61.9 (102.6, 58.8); 96 -> 96 at 2 x 96^2 13.0 (17.4,
+//     25.8), 16 x 128^2 161 (211, 134);
+//   22, 64 x 64, while every CU gets a block: 256 -> 128 at 16 x 32^2 19.6 (66.0; 11:
+//     40.1), 128 -> 128 13.0 (35.7; 18.7), 64 -> 64 at 16 x 64^2 16.6 (31.4; 27.2),
+//     16 x 128^2 66.9 (84.6; 41: 83.9);
+//   11, 32 x 32, the weights of nine steps in flight, below (128 -> 128 at 64^2 8.5,
+//     22: 9.8, k_conv3 18.4) and where the rows leave the LDS no room for more, up
+//     to six blocks a CU: 128 -> 32 at 3 x 128^2, 6 blocks, 37.9 (50.0), but 64 -> 64
+//     at 256^2, 16 blocks, 70.3 (32.6), 64 -> 32, 8 blocks, 37.7 (21.8).
+static int conv_packed_tile(const ConvArgs &a) {
+    if (!conv_direct(a) || conv_lds(a, 1) > kConvLds || !packed_elements(a.C, a.N)) return 0;
+    const int64_t cus = device_cus();
+    auto blocks = [&](int mt, int nt) {
+        return int64_t((a.P + 32 * mt - 1) / (32 * mt)) * ((a.N + 32 * nt - 1) / (32 * nt));
+    };
+    const bool half = a.N <= 32 || (a.N > 64 && a.N <= 96);
+    if (half && conv_lds(a, 4) <= kConvLds && 2 * blocks(4, 1) >= 3 * cus) return 41;
+    if (conv_lds(a, 2) <= kConvLds && blocks(2, 2) >= cus) return 22;
+    return blocks(1, 1) <= 6 * cus ? 11 : 0;
 }
 
 template <int MT, int NT, int D>
@@ -1357,24 +1380,12 @@ static int launch_conv_packed(const ConvArgs &a, hipStream_t s) {
     return launch_status();
 }
 
-static int run_conv_packed(const ConvArgs &a, hipStream_t s) {
-    // us of the whole layer, batch 16 of a 128 x 128 network unless said otherwise,
-    // against the best tile of k_conv3:
-    //   128 pixels x 32 channels while that gives every CU eight blocks: few
-    //     channels, where staging weighs most (32 -> 32 at 128^2: 26.9, 2 x 2
-    //     tiles 31.0, k_conv3 26.8; 96 -> 32: 62.5, 102, 59);
-    //   64 x 64 while every CU gets a block (256 -> 128 at 32^2: 18.9 against
-    //     54, 513 TFLOP/s; 128 -> 128: 13.0 against 31; 64 -> 64 at 64^2: 16.6
-    //     against 27);
-    //   32 x 32 below, the weights of nine steps in flight (128 -> 128 at 16^2: 7.7
-    //     against 15; batch 1, 256 -> 128 at 32^2: 10.7 against 18.3).
-    const int64_t cus = device_cus();
-    auto blocks = [&](int mt, int nt) {
-        return int64_t((a.P + 32 * mt - 1) / (32 * mt)) * ((a.N + 32 * nt - 1) / (32 * nt));
-    };
-    if (a.N <= 96 && conv_lds(a, 4) <= kConvLds && blocks(4, 1) >= 8 * cus) return launch_conv_packed<4, 1, 3>(a, s);
-    if (conv_lds(a, 2) <= kConvLds && blocks(2, 2) >= cus) return launch_conv_packed<2, 2, 3>(a, s);
-    return launch_conv_packed<1, 1, 9>(a, s);
+static int run_conv_packed(const ConvArgs &a, int tile, hipStream_t s) {
+    switch (tile) {
+    case 41: return launch_conv_packed<4, 1, 3>(a, s);
+    case 22: return launch_conv_packed<2, 2, 3>(a, s);
+    default: return launch_conv_packed<1, 1, 9>(a, s);
+    }
 }
 
 extern "C" {
@@ -1385,7 +1396,7 @@ int lbm_nn_packed_fits(int B, int H, int W, int cin, int cout) {
         P * cout >= (int64_t(1) << 31))
         return 0;
     const ConvArgs a{nullptr, nullptr, nullptr, nullptr, nullptr, int(P), H, W, cin, cout, 1, 0, 0};
-    return conv_packed_fits(a);
+    return conv_packed_tile(a) != 0;
 }
 
 int64_t lbm_nn_packed_size(int cin, int cout) {
@@ -1554,7 +1565,7 @@ int lbm_nn_conv3x3_packed(const void *x, int B, int H, int W, int cin, const voi
     if (wp && P * 9 * cin < (int64_t(1) << 31) && P * cout < (int64_t(1) << 31)) {
         const ConvArgs a{static_cast<const uint16_t *>(x), static_cast<const uint16_t *>(wp), y,
                          static_cast<uint16_t *>(yb), bias, int(P), H, W, cin, cout, 1, 0, relu};
-        if (conv_packed_fits(a)) return run_conv_packed(a, as_stream(stream));
+        if (const int tile = conv_packed_tile(a)) return run_conv_packed(a, tile, as_stream(stream));
     }
     return lbm_nn_conv3x3(x, B, H, W, cin, w, cout, bias, y, yb, relu, stream);
 }
@@ -1567,8 +1578,8 @@ int lbm_nn_conv3x3_dgrad_packed(const void *dy, const void *wp, int B, int H, in
     if (P * 9 * cout >= (int64_t(1) << 31) || P * cin >= (int64_t(1) << 31)) return LBM_E_SIZE;
     const ConvArgs a{static_cast<const uint16_t *>(dy), static_cast<const uint16_t *>(wp), dx, nullptr,
                      nullptr, int(P), H, W, cout, cin, -1, 0, 0};
-    if (!conv_packed_fits(a)) return LBM_E_ARG;
-    return run_conv_packed(a, as_stream(stream));
+    const int tile = conv_packed_tile(a);
+    return tile ? run_conv_packed(a, tile, as_stream(stream)) : LBM_E_ARG;
 }
 
 int64_t lbm_nn_gemm_workspace(int M, int N, int ksplit) {

@@ -667,3 +667,58 @@ def test_direct_convolution_block_shapes(gpu, tile, B, H, W, C, N):
     dx = torch.full((P, N), 0.25, device="cuda")
     nat.call("lbm_nn_conv3x3_dgrad_t", _p(x), _p(wt), B, H, W, N, C, _p(dx), 1, sp)
     assert torch.equal(dx, _gemm_dgrad(nat, x, w, B, H, W, C, N))
+
+
+# the block shapes of the packed kernel (32 MT pixels x 32 NT channels), each with
+# pixels and channels that do not fill the last one; the last two have rows that
+# leave the LDS no room for more than 32 pixels
+@pytest.mark.parametrize("tile,B,H,W,C,N", [((4, 1), 3, 129, 131, 32, 3), ((4, 1), 3, 129, 131, 64, 18),
+                                            ((4, 1), 3, 129, 131, 96, 32), ((4, 1), 1, 129, 131, 32, 90),
+                                            ((2, 2), 1, 129, 131, 32, 3), ((2, 2), 2, 100, 101, 96, 32),
+                                            ((2, 2), 2, 90, 92, 32, 50), ((2, 2), 1, 95, 97, 64, 96),
+                                            ((2, 2), 1, 80, 81, 32, 130), ((1, 1), 1, 16, 17, 64, 40),
+                                            ((1, 1), 1, 66, 256, 64, 30), (None, 1, 200, 256, 64, 30)])
+def test_packed_convolution_block_shapes(gpu, tile, B, H, W, C, N):
+    import ctypes
+    nat = _nat()
+    lib = nat.load()
+    cus = torch.cuda.get_device_properties(0).multi_processor_count
+    P, sp = B * H * W, nat.stream_ptr()
+
+    def blocks(mt, nt):
+        return -(-P // (32 * mt)) * -(-N // (32 * nt))
+
+    def room(mt):
+        return (32 * mt + 2 * W + 3) * (2 * C + 16) <= 80 * 1024
+
+    if (N <= 32 or 64 < N <= 96) and room(4) and 2 * blocks(4, 1) >= 3 * cus:
+        chosen = (4, 1)
+    elif room(2) and blocks(2, 2) >= cus:
+        chosen = (2, 2)
+    else:
+        chosen = (1, 1) if room(1) and blocks(1, 1) <= 6 * cus else None
+    print("packed", tile, chosen, B, H, W, C, N, flush=True)
+    assert chosen == tile or cus != 256
+    assert lib.lbm_nn_packed_fits(B, H, W, C, N) == (chosen is not None)
+    rng = np.random.default_rng(C + N + W)
+    x, _ = _bf(rng, (B, H, W, C))
+    bias = torch.as_tensor(rng.normal(size=N).astype(np.float32)).cuda()
+    zero = (ctypes.c_int64 * 1)(0)
+    for transposed in (0, 1):
+        cin, cout = (N, C) if transposed else (C, N)
+        w, _ = _bf(rng, (cout, 3, 3, cin), 0.2)
+        wp = torch.full((int(lib.lbm_nn_packed_size(cin, cout)),), float("nan"), dtype=torch.bfloat16, device="cuda")
+        ci, co = (ctypes.c_int * 1)(cin), (ctypes.c_int * 1)(cout)
+        nat.call("lbm_nn_pack_weights", _p(w), ctypes.addressof(zero), ctypes.addressof(ci), ctypes.addressof(co),
+                 1, transposed, _p(wp), ctypes.addressof(zero), sp)
+        if transposed:
+            dx = torch.full((P, N), float("nan"), device="cuda")
+            status = lib.lbm_nn_conv3x3_dgrad_packed(_p(x), _p(wp), B, H, W, N, C, _p(dx), sp)
+            assert status == (0 if chosen else -3)
+            # dx + 0.25 rounds as the accumulated reference does
+            assert chosen is None or torch.equal(dx + 0.25, _gemm_dgrad(nat, x, w, B, H, W, C, N))
+        else:
+            ye, yeb = _gemm_conv(nat, x, w, B, H, W, C, N, bias, 1)
+            y, yb = torch.full_like(ye, float("nan")), torch.full_like(yeb, float("nan"))
+            nat.call("lbm_nn_conv3x3_packed", _p(x), B, H, W, C, _p(w), _p(wp), N, _p(bias), _p(y), _p(yb), 1, sp)
+            assert torch.equal(y, ye) and torch.equal(yb, yeb)
