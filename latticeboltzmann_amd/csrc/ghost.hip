@@ -98,11 +98,18 @@ __device__ __forceinline__ void sf_eq(T a0, T a1, T a2, T ux, T uy, T e[9]) {
 
 // Density factors of an array density (computed in T): 2 rho / 9 and rho / 36
 // are rho / 18 times powers of two, so they round to the same digits and one
-// division serves all three ...
+// division serves all three, unless 2 rho overflows or a quotient is subnormal
+// (nodes that cleared walls have drained for thousands of steps) ...
 template <typename T>
 __device__ __forceinline__ void eq_of_node(T rho, T ux, T uy, T e[9]) {
-    const T a1 = rho / T(18);
-    sf_eq<T>(T(4) * a1, a1, T(0.5) * a1, ux, uy, e);
+    constexpr T kLeast = sizeof(T) == 8 ? T(0x1p-1016) : T(0x1p-120), kMost = sizeof(T) == 8 ? T(0x1p1022) : T(0x1p126);
+    const T a1 = rho / T(18), m = fabs(rho);
+    T a0 = T(4) * a1, a2 = T(0.5) * a1;
+    if (__builtin_expect(!(m >= kLeast && m <= kMost), 0)) {
+        a0 = T(2) * rho / T(9);
+        a2 = rho / T(36);
+    }
+    sf_eq<T>(a0, a1, a2, ux, uy, e);
 }
 // ... and of the scalar inlet / outlet density, a Python float: the factors
 // are computed in double and then meet the arrays in T.

@@ -241,3 +241,66 @@ def test_step_ends_in_the_buffer_of_single_steps(gpu, flow, nx, ny, steps):
 def test_launch_splits_match_oracle(gpu, flow, tdt, ndt, nx, ny, steps):
     # launches of 4 + 4, 3 + 3 + 2 + 2 (small tiles) and 4 + 4 + 1 + 1 steps
     test_several_steps_per_launch_match_oracle(gpu, flow, tdt, ndt, nx, ny, steps)
+
+
+@pytest.mark.parametrize("tdt,ndt", DT)
+@pytest.mark.parametrize("flow", ["walls", "before", "after"])
+@pytest.mark.parametrize("where", ["smallest", "small", "largest", "mixed"])
+def test_densities_at_the_ends_of_the_type(gpu, tdt, ndt, flow, where):
+    # 2 rho / 9 and rho / 36 where they round as subnormals or overflow, as in ghost
+    # nodes that cleared walls have drained for thousands of steps, beside others
+    from latticeboltzmann_amd import ghost
+    nx, ny, info = 45, 67, np.finfo(ndt)
+    lo, hi = np.log2(float(info.smallest_subnormal)), np.log2(float(info.max))
+    a, b = {"smallest": (lo, lo + 6), "small": (lo, lo + 70), "largest": (hi - 3, hi - 0.1), "mixed": (lo, 1)}[where]
+    r = np.random.default_rng(len(where))
+    rho = (2.0 ** r.uniform(a, b, (nx, ny))).astype(ndt)
+    ux, uy = ((0.03 * r.standard_normal((nx, ny))).astype(ndt) for _ in range(2))
+    rules, pbc, before, after = [], None, None, lambda G: None
+    if flow == "before":
+        pbc, before = ("before", 1.01, 0.99), lambda G: g.pressure_periodic(G, 1.01, 0.99)
+    elif flow == "after":
+        pbc, after = ("after", 1.01, 0.99), lambda G: g.pressure_periodic_after(G, 1.01, 0.99)
+    else:
+        rules, after = ghost.side_walls(nx, ny, 0.05), lambda G: g.bounce_back_walls(G, 0.05)
+    with np.errstate(all="ignore"):
+        start = g.equilibrium(rho, ux, uy)
+        for steps in (1, 4, 7):
+            print("ends", tdt, flow, where, steps, flush=True)
+            lat = ghost.GhostLattice(nx, ny, 1.3, rules, pbc, dtype=tdt).load(start)
+            mom = lat.moment_buffers()
+            lat.step(steps, moments=mom)
+            G = start.copy()
+            for _ in range(steps):
+                if before:
+                    before(G)
+                g.stream(G)
+                after(G)
+                omom = g.collide(G, 1.3)
+            assert np.array_equal(lat.populations(), G, equal_nan=True)
+            for x, y in zip(mom, omom):
+                assert np.array_equal(x.cpu().numpy(), y, equal_nan=True)
+
+
+def test_drained_ghost_nodes_match_oracle(gpu):
+    # clearing walls: after 6000 steps the cleared nodes' densities are subnormal
+    from latticeboltzmann_amd import ghost
+    nx, ny, steps = 24, 20, 6000
+    r = np.random.default_rng(0)
+    start = g.at_rest(nx, ny) + 1e-3 * r.standard_normal((9, nx, ny))
+    lat = ghost.GhostLattice(nx, ny, 0.5, ghost.pulse_walls(nx, ny, True)).load(start)
+    lat.step(steps)
+    G, m = start.copy(), nx - 1
+    with np.errstate(all="ignore"):
+        for _ in range(steps):
+            g.stream(G)
+            for ch, src in ((1, 3), (5, 7), (8, 6)):
+                G[ch, 1] = G[src, 0]
+            G[[3, 7, 6], 0] = 0
+            for ch, src in ((3, 1), (6, 8), (7, 5)):
+                G[ch, m - 1] = G[src, m]
+            G[[1, 8, 5], m] = 0
+            g.collide(G, 0.5)
+    rho = np.abs(G.sum(0))
+    assert rho[rho > 0].min() < np.finfo(np.float64).tiny
+    assert np.array_equal(lat.populations(), G, equal_nan=True)
