@@ -304,3 +304,36 @@ def test_drained_ghost_nodes_match_oracle(gpu):
     rho = np.abs(G.sum(0))
     assert rho[rho > 0].min() < np.finfo(np.float64).tiny
     assert np.array_equal(lat.populations(), G, equal_nan=True)
+
+
+@pytest.mark.parametrize("tdt,ndt", DT)
+@pytest.mark.parametrize("layout", ["rows", "soa"])
+@pytest.mark.parametrize("mode", ["before", "after"])
+@pytest.mark.parametrize("nx", [3, 4, 5, 9, 40])
+def test_single_steps_near_inlet_and_outlet(gpu, tdt, ndt, layout, mode, nx):
+    # grids of nothing but columns near the inlet and outlet, and rules whose
+    # sources lie up to the whole grid away
+    from latticeboltzmann_amd import ghost
+    ny, far = 600, nx - 1
+    rules = [ghost.Rule(0, 1, 2, 590, 1, 3, far, 4), ghost.Rule(far, nx, 3, 599, 6, 8, -far, -2)]
+    args = (1.01, 0.99)
+    r = np.random.default_rng(nx)
+    rho = (1 + 0.02 * r.standard_normal((nx, ny))).astype(ndt)
+    ux, uy = ((0.03 * r.standard_normal((nx, ny))).astype(ndt) for _ in range(2))
+    lat = ghost.GhostLattice(nx, ny, 1.3, rules, (mode,) + args, dtype=tdt, layout=layout)
+    lat.init_equilibrium(rho, ux, uy)
+    mom = lat.moment_buffers()
+    G = g.equilibrium(rho, ux, uy)
+    for _ in range(3):
+        print("near", tdt, layout, mode, nx, flush=True)
+        lat.step(1, moments=mom)
+        if mode == "before":
+            g.pressure_periodic(G, *args)
+        g.stream(G)
+        if mode == "after":
+            g.pressure_periodic_after(G, *args)
+        a = G[3, far, 6:594].copy()
+        b = G[8, 0, 1:597].copy()
+        G[1, 0, 2:590], G[6, far, 3:599] = a, b
+        omom = g.collide(G, 1.3)
+        same(lat, mom, G, omom)
