@@ -829,8 +829,18 @@ template <typename T>
 int launch_ghost_step(const T *src, T *dst, int layout, const GhostParams &p, T *rho, T *ux, T *uy,
                       hipStream_t s) {
     const dim3 grid(unsigned((p.ny + kGhostBlock - 1) / kGhostBlock), unsigned(p.nx));
+    // HBM-bound in FP64, three blocks a CU instead of four read fewer rows at a time
+    // (the LDS they reserve is not used).  us a step of the sliding lid, four / three:
+    // 1500 x 4000 162 / 154, 4098^2 467 / 448, 6000 x 3000 478 / 462, 6000^2 996 / 973;
+    // but 2500 x 2001, half in the last-level cache, 143 / 145, 8192^2 1712 / 1752, short
+    // rows (16000 x 1000) 433 / 450, FP32 3000 x 6000 246 / 244, 4000^2 210 / 247.
+    // The kernel with inlet and outlet has registers for two blocks anyway.
+    const int64_t nodes = int64_t(p.nx) * p.ny;
+    const bool three = sizeof(T) == 8 && p.pbc_mode == LBM_PBC_NONE && p.ny >= 1500 &&
+                       nodes >= 5500000 && nodes <= 40000000;
+    const unsigned lds = three ? 52 * 1024 : 0;
     auto launch = [&](auto kernel) {
-        hipLaunchKernelGGL(kernel, grid, dim3(kGhostBlock), 0, s, src, dst, p, rho, ux, uy);
+        hipLaunchKernelGGL(kernel, grid, dim3(kGhostBlock), lds, s, src, dst, p, rho, ux, uy);
     };
     const bool rows = layout == LBM_LAYOUT_ROWS;
     if (p.pbc_mode == LBM_PBC_NONE) {
