@@ -1003,16 +1003,16 @@ bool launch_ghost_multi(const T *src, T *dst, int layout, const GhostParams &p, 
 
 // Tile shapes, four steps per launch.  VALU-bound at large grids, like the
 // cavity's tiles, so the widest tile that leaves two blocks per CU:
-// 1: flows that read their neighbours only; 4098^2 FP64 sliding lid 176 us a
-//    step (95 GLUPS), 452 us with one step per launch (HBM-bound, 5.4 TB/s);
+// 1: flows that read their neighbours only; 4098^2 FP64 sliding lid 173 us a
+//    step (97 GLUPS), 452 us with one step per launch (HBM-bound, 5.4 TB/s);
 // 0: room for the inlet and outlet columns, 512 threads because their
 //    arithmetic spills at the 80 registers that 768 leave: 4098^2 FP64 canal
-//    245 us a step against 455 with one step per launch, 1000 x 1501 24 us
+//    253 us a step against 425 with one step per launch, 1000 x 1501 24 us
 //    against 33 with 768 threads;
-// 2: grids of fewer than two 22 x 32 tiles per CU: more and smaller blocks, all
-//    latency; 102 x 52 FP64 canal 4.0 us a step against 13.9, where the inlet
-//    and outlet take 1.9 us of it and the rules 1.0.  Six or eight steps per
-//    launch (4.4, 4.6 us), also with one loop body for all steps, gave nothing.
+// 2: grids of so few tiles of shape 0 that half of the CUs had none: more and
+//    smaller blocks, all latency; 102 x 52 FP64 canal 4.1 us a step against 12.0,
+//    where the inlet and outlet take 1.9 us of it and the rules 1.0.  Six or eight
+//    steps per launch (4.4, 4.6 us), also with one loop body for all steps, gave nothing.
 template <typename T>
 bool ghost_multi(int shape, const T *src, T *dst, int layout, const GhostParams &p, const GhostPlan &w,
                  int K, T *rho, T *ux, T *uy, hipStream_t s, bool check) {
@@ -1037,10 +1037,19 @@ int ghost_run(T *a, T *b, int64_t nx, int64_t ny, int layout, double omega, cons
     GhostPlan w;
     int shape = -1;
     if (steps > 1 && ghost_plan(p, w)) {
-        const int64_t tiles = ((nx + 21) / 22) * ((ny + 31) / 32);
-        // small grids first try shape 2; wide-reading flows do not fit shape 1,
-        // and narrow or crowded grids may fit shape 2 only
-        const int order[3] = {tiles < 2 * int64_t(device_cus()) ? 2 : 1, 0, 2};
+        // us a step, FP64 (FP32), shapes 0 / 1 / 2: canal 102 x 52, 12 tiles of shape 0,
+        // 5.5 / - / 4.1 (4.4 / 3.9), 200^2, 84 tiles, 5.4 / - / 4.5 (4.4 / 4.3), 300^2,
+        // 180 tiles, 5.4 / - / 6.4 (4.4 / 6.0), 600^2 8.2 / - / 16.5 (6.5 / 14.9); lid
+        // 200^2 3.3 / 3.6 / 3.0 (2.9 / 3.1 / 2.6), 300^2 3.4 / 3.7 / 4.3 (3.0 / 3.2 /
+        // 3.1), 500^2 4.9 / 5.3 / 7.6 (3.6 / 4.2 / 5.7).  Shape 1 where it saves a round
+        // of two blocks a CU: 1000 x 300, 590 tiles against 460, 6.0 / 5.3 / 8.4 (4.1 /
+        // 3.9 / 6.3), but 600^2, 684 against 532, 6.6 / 7.2 / 9.9 (4.1 / 5.2 / 6.9).
+        const int64_t cus = device_cus();
+        const int64_t tiles0 = ((nx + 16) / 17) * ((ny + 31) / 32), tiles1 = ((nx + 21) / 22) * ((ny + 31) / 32);
+        auto rounds = [&](int64_t tiles) { return (tiles + 2 * cus - 1) / (2 * cus); };
+        // wide-reading flows do not fit shape 1, and narrow or crowded grids may
+        // fit shape 2 only
+        const int order[3] = {2 * tiles0 <= cus ? 2 : (rounds(tiles1) < rounds(tiles0) ? 1 : 0), 0, 2};
         for (int k = 0; k < 3 && shape < 0; ++k)
             if (ghost_multi<T>(order[k], a, b, layout, p, w, kGhostMaxK, rho, ux, uy, s, true))
                 shape = order[k];
