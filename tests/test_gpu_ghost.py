@@ -337,3 +337,44 @@ def test_single_steps_near_inlet_and_outlet(gpu, tdt, ndt, layout, mode, nx):
         G[1, 0, 2:590], G[6, far, 3:599] = a, b
         omom = g.collide(G, 1.3)
         same(lat, mom, G, omom)
+
+
+@pytest.mark.parametrize("tdt,ndt", DT)
+@pytest.mark.parametrize("mode", ["before", "after"])
+@pytest.mark.parametrize("nx,ny,steps", [(45, 67, 8), (45, 67, 7), (45, 67, 10), (120, 130, 8), (361, 1067, 8)])
+def test_wall_density_rules_with_inlet_and_outlet(gpu, tdt, ndt, mode, nx, ny, steps):
+    # the lid weighted by the wall's density where an inlet and outlet are, over all
+    # columns, from the inlet and outlet columns and from one beside them, and from
+    # two columns away; several steps a launch against the oracle
+    from latticeboltzmann_amd import _native as nat
+    from latticeboltzmann_amd import ghost
+    k = nat.RULE_LID_RHO
+    rules = [ghost.Rule(0, nx, ny - 2, ny - 1, 7, 5, 0, 1, k, -0.02),
+             ghost.Rule(0, nx, ny - 2, ny - 1, 8, 6, 0, 1, k, 0.02),
+             ghost.Rule(1, 2, 3, ny - 6, 4, 3, -1, 0, k, 0.01),         # source: the inlet
+             ghost.Rule(nx - 2, nx - 1, 3, ny - 6, 4, 1, 1, 0, k, 0.01),  # the outlet
+             ghost.Rule(4, 5, 3, ny - 6, 4, 2, -2, 0, k, 0.03),         # column 2, two away
+             ghost.Rule(2, 3, 4, 9, 4, 0, -1, 1, k, 0.01)]              # column 1, beside the inlet
+    args = (1.01, 0.99)
+    r = np.random.default_rng(nx + steps)
+    rho = (1 + 0.02 * r.standard_normal((nx, ny))).astype(ndt)
+    ux, uy = ((0.03 * r.standard_normal((nx, ny))).astype(ndt) for _ in range(2))
+    print("wall density", tdt, mode, nx, ny, steps, flush=True)
+    lat = ghost.GhostLattice(nx, ny, 1.3, rules, (mode,) + args, dtype=tdt,
+                             layout="soa" if steps == 7 else "rows")
+    lat.init_equilibrium(rho, ux, uy)
+    mom = lat.moment_buffers()
+    lat.step(steps, moments=mom)
+    G = g.equilibrium(rho, ux, uy)
+    for _ in range(steps):
+        if mode == "before":
+            g.pressure_periodic(G, *args)
+        g.stream(G)
+        if mode == "after":
+            g.pressure_periodic_after(G, *args)
+        for q in rules:
+            s = G[:, q.x0 + q.dx:q.x1 + q.dx, q.y0 + q.dy:q.y1 + q.dy]
+            wall = 2.0 * (s[2] + s[5] + s[6]) + s[0] + s[1] + s[3]
+            G[q.ch, q.x0:q.x1, q.y0:q.y1] = s[q.src_ch] + q.coef * wall
+        omom = g.collide(G, 1.3)
+    same(lat, mom, G, omom)
