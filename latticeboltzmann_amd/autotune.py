@@ -131,6 +131,23 @@ def step_variant(nx, ny, dtype, layout, bc, reps=10, use_cache=True):
                         reps=reps, use_cache=use_cache)
 
 
+def multi_candidates(nx, ny, info, cus):
+    """The variants of ``info`` (variant: steps, least nx, least ny) worth timing on
+    an nx x ny grid: those that fit, but tiles of at most 16 columns only up to four
+    a CU.  There they win (500^2 FP64, 1024 tiles, 3.66 us a step against 4.17);
+    beyond, they lose by less than the spread of a short timing (933^2 8.91 against
+    8.35) and were picked now and then."""
+    out = []
+    for v, (k, mnx, mny) in info.items():
+        rows, cols = mnx - 2 * k, mny - 2 * k
+        if nx < mnx or ny < mny:
+            continue
+        if 0 < cols <= 16 and -(-nx // rows) * -(-ny // cols) > 4 * cus:
+            continue
+        out.append(v)
+    return out
+
+
 def multi_variant(nx, ny, dtype, layout, bc, reps=10, use_cache=True):
     """Autotuned variant of the multi-step kernel (``lbm_step_multi_*``): the
     (steps per launch, tile) shape with the least time per step, or None when
@@ -138,7 +155,8 @@ def multi_variant(nx, ny, dtype, layout, bc, reps=10, use_cache=True):
     from . import kernels
     n_var = nat.load().lbm_step_multi_variant_count()
     info = {v: kernels.step_multi_info(v) for v in range(n_var)}
-    fits = [v for v, (k, mnx, mny) in info.items() if nx >= mnx and ny >= mny]
+    cus = torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count
+    fits = multi_candidates(nx, ny, info, cus)
     if not fits:
         return None
 

@@ -254,3 +254,19 @@ def test_packing_leaves_out_layers_beyond_the_packed_kernels(cin, cout, transpos
     small = lib.lbm_nn_unet_workspace(1, 2, 2, 32, ctypes.addressof(widths), 1, 32, 3)
     large = lib.lbm_nn_unet_workspace(1, 2, 2, 32, ctypes.addressof(widths), 1, 16384, 3)
     assert 0 < small < large < small + (1 << 25)
+
+
+def test_small_tiles_are_tuned_on_small_grids_only():
+    from latticeboltzmann_amd import _native as nat
+    from latticeboltzmann_amd import kernels
+    from latticeboltzmann_amd.autotune import multi_candidates
+    info = {v: kernels.step_multi_info(v) for v in range(nat.load().lbm_step_multi_variant_count())}
+    small = {v for v, (k, mnx, mny) in info.items() if 0 < mny - 2 * k <= 16}
+    assert len(small) == 3
+    assert small <= set(multi_candidates(256, 256, info, 256))
+    for nx, ny in ((933, 933), (2048, 2048), (100, 6000)):
+        got = set(multi_candidates(nx, ny, info, 256))
+        assert not got & small
+        # the others are those that fit
+        assert got == {v for v, (k, mnx, mny) in info.items() if nx >= mnx and ny >= mny} - small
+    assert multi_candidates(15, 15, info, 256) == []
