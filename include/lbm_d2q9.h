@@ -89,7 +89,8 @@ int lbm_stream_periodic(const void *src, void *dst, int64_t nx, int64_t ny,
 
 /* The same in place on f[9][nx][ny] (PyLB.stream modifies its argument).  scratch:
  * lbm_stream_inplace_scratch(nx, ny, walls) elements of f's type, walls = 1 for the
- * cavity form; it must not overlap f.  Element sizes 1, 2, 4 and 8.           */
+ * cavity form; it must not overlap f.  Element sizes 1, 2, 4 and 8.  LBM_E_SIZE for
+ * grids past one launch (from 7 million rows), which the form above streams.  */
 int64_t lbm_stream_inplace_scratch(int64_t nx, int64_t ny, int walls);
 int lbm_stream_inplace(void *f, int64_t nx, int64_t ny, int elem_bytes, void *scratch, void *stream);
 int lbm_stream_bounce_back_inplace_f64(double *f, int64_t nx, int64_t ny, double u0, double *scratch,
@@ -97,7 +98,7 @@ int lbm_stream_bounce_back_inplace_f64(double *f, int64_t nx, int64_t ny, double
 int lbm_stream_bounce_back_inplace_f32(float *f, int64_t nx, int64_t ny, float u0, float *scratch,
                                        void *stream);
 
-/* K full time steps src -> dst in one launch (temporal blocking, K = 2..8
+/* K full time steps src -> dst in one launch (temporal blocking, K = 2..6
  * fixed by the variant).  Tile variants: each block computes the first K-1
  * steps of its tile and a shrinking halo in LDS and writes only the last.
  * Sweep variants: each wave walks a strip of 64 columns along x and keeps the
@@ -385,6 +386,8 @@ int lbm_nn_conv3x3(const void *x, int B, int H, int W, int cin, const void *w, i
 int lbm_nn_conv3x3_wgrad_splits(int B, int H, int W, int cin, int cout);
 int lbm_nn_conv3x3_wgrad(const void *x, const void *dy, int B, int H, int W, int cin, int cout,
                          float *dw, int ksplit, float *work, void *stream);
+/* The data gradient as a general GEMM on flipped weights: no network call takes it,
+ * the tests compare the other forms with it.                                  */
 int lbm_nn_conv3x3_flip_weights(const void *w, int cin, int cout, void *wf, void *stream);
 int lbm_nn_conv3x3_dgrad(const void *dy, const void *wf, int B, int H, int W, int cin, int cout,
                          float *dx, int accumulate, void *stream);
@@ -392,10 +395,10 @@ int lbm_nn_conv3x3_dgrad(const void *dy, const void *wf, int B, int H, int W, in
  * fragments are loaded: lbm_nn_pack_weights packs the BF16 weights of n layers
  * (element offsets from[] into w, to[] into out, multiples of 8; packed size of a
  * layer: lbm_nn_packed_size) in one launch, for the forward pass or (transposed)
- * the data gradient; layers whose cin (transposed: cout) is no multiple of 32 are
- * left out.  conv3x3_packed takes both forms of the weights and the packed one
+ * the data gradient; layers whose cin (transposed: cout) is no multiple of 32, or
+ * whose packed weights would pass 2^31 bytes, are left out.  conv3x3_packed takes both forms of the weights and the packed one
  * (wp, nullable) where it applies; dgrad_packed returns LBM_E_ARG where it does
- * not.  Results are the bits of conv3x3 and dgrad.                           */
+ * not (lbm_nn_packed_fits, of channels summed and computed).  Results are the bits of conv3x3 and dgrad.                           */
 #define LBM_NN_MAX_LAYERS 32
 int64_t lbm_nn_packed_size(int cin, int cout);
 int lbm_nn_packed_fits(int B, int H, int W, int cin, int cout); /* 1 or 0 */

@@ -107,7 +107,7 @@ __global__ __launch_bounds__(BS) void k_step(const T *__restrict__ src, T *__res
     }
 }
 
-// K fused steps per launch (temporal blocking, K = 2..8), src -> dst.
+// K fused steps per launch (temporal blocking, K = 2..6), src -> dst.
 // Block b owns a TR x TC tile of nodes.  Phase 1 computes step 1 on the tile
 // and a halo ring K-1 nodes deep, at wrapped global coordinates, with the
 // single-step node code (pull from src, walls, collide), into LDS; each later
@@ -251,7 +251,7 @@ __global__ __launch_bounds__(BS) void k_stepk(const T *__restrict__ src, T *__re
                                                   int nx, int ny, Layout L, int ntc, int ntiles,
                                                   T omega, T u0, T *__restrict__ rho_o,
                                                   T *__restrict__ ux_o, T *__restrict__ uy_o) {
-    static_assert(K >= 2 && K <= 8, "2 to 8 steps per launch");
+    static_assert(K >= 2 && K <= 6, "2 to 6 steps per launch");
     constexpr int NA = (TR + 2 * (K - 1)) * (TC + 2 * (K - 1));  // the phase-1 ring, the largest
     __shared__ T sa[9 * NA];
     const int tile = xcd_tile(ntiles);
@@ -1007,10 +1007,13 @@ template <typename T>
 inline int default_multi_shape(int64_t nx, int64_t ny) {
     if (nx * ny >= kLargeGridNodes) return kLargeGridMultiShape;
     // Four steps a launch: six gain little (256^2: 1.62 us a step against 1.71) and
-    // leave up to five single steps.  8 x 8 tiles while each has a CU of its own
-    // (128^2: 1.28 us against 1.59 on 16 x 16 and 2.48 on 22 x 32); 16 x 16 while
-    // 22 x 32 tiles would leave half of the CUs idle (256^2: 1.71 against 2.56; at
-    // 384^2, 216 tiles of 22 x 32, they lose 2.75 to 2.55).
+    // leave up to five single steps.  8 x 8 tiles while each has a CU of its own, 16 x
+    // 16 while 22 x 32 tiles would leave half of the CUs idle.  us a step, FP64 (FP32),
+    // on 8 x 8 / 16 x 16 / the tile default: 64^2 1.30 / 1.65 / 2.50 (1.20 / 1.39 /
+    // 2.05), 128^2 1.32 / 1.62 / 2.50 (1.23 / 1.40 / 2.04), 160^2 1.50 / 1.69 / 2.52
+    // (1.29 / 1.43 / 2.05), 256^2 2.03 / 1.72 / 2.59 (1.70 / 1.47 / 2.11), 64 x 1024
+    // 2.12 / 1.83 / 2.59 (1.65 / 1.52 / 2.19).  FP64 16 x 16 tiles gain nothing from
+    // 360^2 (2.59 / 2.61; 400^2 2.77 / 2.63), FP32 ones still 8 % there (2.03 / 2.21).
     constexpr bool f32 = sizeof(T) == sizeof(float);
     const int64_t cus = device_cus();
     if (nx >= (f32 ? 28 : 30) && ny >= 40) {  // grids that the tile default takes

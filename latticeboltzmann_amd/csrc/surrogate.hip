@@ -862,7 +862,8 @@ __global__ __launch_bounds__(256) void k_transpose_weights(const uint16_t *__res
 }
 
 // Weights W[cout][tap][cin] -> Wf[tap][cout][cin] (BF16): the B operand of the
-// data-gradient GEMM, dX[p][c] = sum over (tap, co) of dY[p - tap][co] Wf[tap][co][c].
+// data gradient as a general GEMM (the form that the others are tested against),
+// dX[p][c] = sum over (tap, co) of dY[p - tap][co] Wf[tap][co][c].
 __global__ __launch_bounds__(256) void k_flip_weights(const uint16_t *__restrict__ w, int cin,
                                                       int cout, uint16_t *__restrict__ wf) {
     const int i = blockIdx.x * 256 + threadIdx.x;  // over tap, cout, cin

@@ -2,7 +2,7 @@
 
 This is the engine behind the reference's driver loops
 (``cavity_opt1.py:338-347``, ``shear_wave_opt1.py:170-174``): two population
-buffers ping-pong through the fused pull stream-collide kernels, up to eight
+buffers ping-pong through the fused pull stream-collide kernels, up to six
 steps per launch, on one stream; one native call issues the launches of a
 ``step``.  By default the populations are kept in the
 row-interleaved layout ``f[k][i][l]`` (nine channel segments of an x-row
@@ -52,7 +52,7 @@ class Lattice:
         autotuned; "auto" also tunes the multi-step kernel's shape).
     layout : ``"rows"`` (default) or ``"soa"`` (the reference's f[i][k][l]).
     multi_step : advance runs of K steps with the temporally blocked
-        multi-step kernel (``lbm_step_multi_*``, K = 2..8 per launch, bitwise
+        multi-step kernel (``lbm_step_multi_*``, K = 2..6 per launch, bitwise
         equal to K single steps) where the grid is large enough for its tiles.
     """
 
