@@ -83,8 +83,9 @@ def best_variant(kernel, nx, ny, dtype, layout, bc, make_launch, variants, reps=
     the launch times to the times compared (e.g. per step).
     """
     dev = torch.cuda.get_device_name(torch.cuda.current_device())
+    # the last field names the way of timing: choices made another way are not reused
     key = "|".join([nat.build_id(), dev, kernel, str(dtype), str(layout), str(bc),
-                    size_class(nx, ny)])
+                    size_class(nx, ny), "close ones again"])
     with _LOCK:
         if key in _MEMO:
             return _MEMO[key]
@@ -93,9 +94,17 @@ def best_variant(kernel, nx, ny, dtype, layout, bc, make_launch, variants, reps=
             _MEMO[key] = entries[key]["variant"]
             return _MEMO[key]
     launch = make_launch(nx, ny)
-    times = time_variants(launch, list(variants), reps=reps)
-    if normalize is not None:
-        times = normalize(times)
+    normalize = normalize or (lambda t: t)
+    timed = time_variants(launch, list(variants), reps=reps)
+    times = normalize(timed)
+    # ten launches of some 10 us are easily disturbed (256^2 FP64: a variant of 1.83 us
+    # a step measured 2.30, and the choice is kept), so the close ones are timed
+    # twice again, each at its best
+    near = [v for v in times if times[v] <= 1.3 * min(times.values())]
+    for _ in range(2 if len(near) > 1 else 0):
+        again = time_variants(launch, near, reps=reps)
+        timed.update((v, min(timed[v], again[v])) for v in near)
+    times = normalize(timed)
     best = min(times, key=times.get)
     with _LOCK:
         _MEMO[key] = best

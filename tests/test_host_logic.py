@@ -270,3 +270,29 @@ def test_small_tiles_are_tuned_on_small_grids_only():
         # the others are those that fit
         assert got == {v for v, (k, mnx, mny) in info.items() if nx >= mnx and ny >= mny} - small
     assert multi_candidates(15, 15, info, 256) == []
+
+
+def test_tuner_times_close_variants_again(monkeypatch, tmp_path):
+    from latticeboltzmann_amd import _native as nat
+    from latticeboltzmann_amd import autotune
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "get_device_name", lambda d: "none")
+    monkeypatch.setattr(nat, "build_id", lambda: "0")
+    monkeypatch.setenv("LBM_TUNE_CACHE", str(tmp_path / "tune.json"))
+    monkeypatch.setattr(autotune, "_MEMO", {})
+    true = {1: 4.0, 2: 4.4, 3: 9.0, 4: 8.0}  # per launch; variant 4 makes two steps
+    rounds = []
+
+    def timed(launch, variants, reps=10, warmup=2):
+        rounds.append(list(variants))
+        slow = 1.25 if len(rounds) == 1 else 1.0  # the first timing of variant 1 was disturbed
+        return {v: true[v] * (slow if v == 1 else 1.0) for v in variants}
+
+    monkeypatch.setattr(autotune, "time_variants", timed)
+    best = autotune.best_variant("k", 64, 64, "f64", 0, 0, lambda nx, ny: None, [1, 2, 3])
+    assert best == 1 and rounds == [[1, 2, 3], [1, 2], [1, 2]]
+    del rounds[:]
+    best = autotune.best_variant("m", 64, 64, "f64", 0, 0, lambda nx, ny: None, [2, 3, 4],
+                                 normalize=lambda t: {v: x / (2 if v == 4 else 1) for v, x in t.items()})
+    assert best == 4 and rounds == [[2, 3, 4], [2, 4], [2, 4]]
+    assert autotune.best_variant("k", 64, 64, "f64", 0, 0, None, [1, 2, 3]) == 1  # kept
