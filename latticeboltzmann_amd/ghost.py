@@ -244,7 +244,9 @@ class GhostLattice:
 
     def step(self, n=1, moments=None):
         """n full steps (walls, then collide); ``moments`` receives the
-        pre-collision moments of the last one."""
+        pre-collision moments of the last one.  The state ends in the buffer where
+        n single-step launches would leave it: ``f`` itself for an even n, which a
+        captured graph needs."""
         n = operator.index(n)
         if n > 0:
             rho, ux, uy = moments if moments is not None else (None, None, None)

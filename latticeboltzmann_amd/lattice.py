@@ -237,6 +237,7 @@ class StepGraph:
 
     def __init__(self, lat, n, enabled=True):
         self.lat, self.n = lat, int(n)
+        # a lattice without launches() ends where n single steps would (GhostLattice)
         swaps = lat.launches(self.n) if hasattr(lat, "launches") else self.n
         self.enabled = bool(enabled) and swaps % 2 == 0
         self.graph = None

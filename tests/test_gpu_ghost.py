@@ -378,3 +378,12 @@ def test_wall_density_rules_with_inlet_and_outlet(gpu, tdt, ndt, mode, nx, ny, s
             G[q.ch, q.x0:q.x1, q.y0:q.y1] = s[q.src_ch] + q.coef * wall
         omom = g.collide(G, 1.3)
     same(lat, mom, G, omom)
+
+
+@pytest.mark.parametrize("tdt,ndt", DT)
+@pytest.mark.parametrize("nx,ny,steps", [(329, 999, 11), (700, 500, 7), (120, 517, 6), (250, 250, 11)])
+@pytest.mark.parametrize("flow", ["lid", "couette", "sides", "canal"])
+def test_tile_shapes_match_oracle(gpu, flow, tdt, ndt, nx, ny, steps):
+    # on 256 CUs: 22 x 32 tiles (inlet and outlet: 17 x 32) on the first two grids,
+    # 17 x 32 on the third, 6 x 16 on the last; launches of 4 + 4 + 3, 4 + 2 + 1 and 4 + 2
+    test_several_steps_per_launch_match_oracle(gpu, flow, tdt, ndt, nx, ny, steps)
